@@ -737,6 +737,9 @@ sa3k_block_ws* block_ws_build(const sa3k_block_config& cfg, int B, int S, int Ct
 void block_prepare(sa3k_ctx* ctx, sa3k_block* b, const float* const* A, const float* const* Bm,
                    const float* const* mag, float scale, int dora) {
     SA3K_REQUIRE(b && A && Bm && (!dora || mag), "null adapter arrays");
+    // all of the block's linears in one launch: seven of their own took 45 + 8 us each at 1536
+    // columns, most of it their workgroups' chains of memory round trips
+    if (lin_prepare_merged(ctx, b->L, NT, A, Bm, mag, b->bnsq, scale, dora)) return;
     for (int t = 0; t < NT; ++t)
         chk(ctx, sa3k_lin_prepare(ctx, b->L[t], A[t], Bm[t], scale, dora, dora ? mag[t] : nullptr,
                                   dora ? b->bnsq[t] : nullptr));

@@ -33,6 +33,11 @@ LinGroup* lin_group_create(sa3k_ctx* ctx, sa3k_lin* const* lins, int n, const fl
 // the grouped equivalent of sa3k_lin_prepare on every member
 void lin_group_prepare(sa3k_ctx* ctx, LinGroup* g);
 void lin_group_free(LinGroup* g);
+// sa3k_lin_prepare on up to 8 bf16 linears of one rank in one launch (the merged refresh), with
+// their descriptors as kernel arguments; false, with nothing done, where they are not eligible.
+// mag / bnsq: one per linear for dora.
+bool lin_prepare_merged(sa3k_ctx* ctx, sa3k_lin* const* lins, int n, const float* const* A, const float* const* B,
+                        const float* const* mag, const float* const* bnsq, float scale, int dora);
 // A short role name ("qkv", "ff.out", ...) appended to the linear's profiler scope names, so a
 // per-kernel profile separates the projections (no effect while profiling is off).
 void lin_set_tag(sa3k_lin* l, const char* tag);

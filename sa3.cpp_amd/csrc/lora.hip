@@ -66,10 +66,6 @@ struct sa3k_lin {
     int merged = 0;
     void* Wm = nullptr;                 // [out][in] bf16 W_eff
     void* Wmt = nullptr;                // [in][out] bf16 W_eff^T
-    sa3k::LinGroup* solo = nullptr;     // one-member group refreshing a separately prepared linear
-    const float* solo_key[4] = {};      // its A, B, magnitude, base_norm_sq pointers
-    float solo_s = 0.0f;
-    int solo_dora = -1;
 };
 
 namespace {
@@ -862,7 +858,6 @@ constexpr unsigned kExtAc = 1, kExtD = 2, kExtWm = 4, kExtU = 8, kExtHc = 16;
 
 void free_lin(sa3k_lin* L) {
     if (!L) return;
-    if (L->solo) lin_group_free(L->solo);
     for (void* p : {L->Xb, L->At, L->Bc, L->Bt, (void*)L->Pt, (void*)L->G, (void*)L->BG, (void*)L->nsq, L->dU,
                     L->sdUB, (void*)L->gd, (void*)L->gn, L->Ax, L->A2x, (void*)L->red, L->Wmt})
         if (p) (void)hipFree(p);
@@ -1249,51 +1244,92 @@ struct PrepDesc {
     const void* Wsrc;
     const void* Wsc;
     int wtype;
+    int msplit;                        // column splits of each 64-row block (merge_splits)
     bf16 *Wm, *Wmt;
 };
 
+// The members of a refresh as its kernels see them: a table in device memory with the member of
+// every block (large groups), or the descriptors themselves as kernel arguments (up to kInlineMax
+// members, in block order in every stage): nothing to upload, wait for or keep between calls.
+constexpr int kInlineMax = 8;
+struct PrepTable {
+    const PrepDesc* ds;
+    const int* block_member;
+    __device__ __forceinline__ const PrepDesc& find(int, int b) const { return ds[block_member[b]]; }
+};
+struct PrepInline {
+    PrepDesc ds[kInlineMax];
+    int n;
+    __device__ __forceinline__ const PrepDesc& find(int stage, int b) const {
+        int m = 0;
+        for (int k = 1; k < n; ++k)
+            if (b >= ds[k].blk0[stage]) m = k;
+        return ds[m];
+    }
+};
+
+typedef unsigned u32x4u __attribute__((ext_vector_type(4), aligned(4)));   // adapters are only 4-byte aligned
+__device__ __forceinline__ f32x4 ldg_f4(const float* p) {
+    return __builtin_bit_cast(f32x4, *(__attribute__((address_space(1))) const u32x4u*)p);
+}
+
 // Ac/At/Bc/Bt from A and B. A block converts one 64-wide tile: columns [64t, 64t + 64) of A
 // (all r rows) for its first ceil(in/64) blocks, then rows [64t, 64t + 64) of B (all r columns).
-// The copies in the source layout are written as read; the transposed copies go through LDS so
-// every store is a contiguous row (a direct transposed store touches one cache segment per value).
+// Each of the 256 threads takes 8 consecutive ranks or columns, so every global access is 16 or 32
+// bytes a thread: the copies in the source layout are written as read, the transposed ones go
+// through LDS ([line][element], padded). HBM-bound: 8 bytes a parameter (bf16 copies); a DiT's 38.4 M
+// parameters added 127 us to the refresh with one element a thread and access, 39 us this way.
+constexpr int kConvPitch = 72;   // elements per line: 64 columns of A or 32 ranks of a row of B, padded
 template <class CT>
-__global__ __launch_bounds__(kThreads) void group_convert_kernel(const PrepDesc* __restrict__ ds,
-                                                                 const int* __restrict__ block_member, int r) {
-    const PrepDesc& q = ds[block_member[blockIdx.x]];
-    __shared__ CT tile[64][34];   // [tile index][rank], padded
+__device__ __forceinline__ void store8(CT* dst, const CT (&v)[8]) {
+    struct alignas(16) Q { CT e[16 / sizeof(CT)]; };
+    constexpr int N = (int)(16 / sizeof(CT));
+#pragma unroll
+    for (int k = 0; k < 8; k += N) {
+        Q q;
+#pragma unroll
+        for (int e = 0; e < N; ++e) q.e[e] = v[k + e];
+        *reinterpret_cast<Q*>(dst + k) = q;
+    }
+}
+template <class CT>
+__device__ __forceinline__ void convert_tile(const PrepDesc& q, int t, int r, CT* tile) {
     CT* const Ac = static_cast<CT*>(q.Ac);
     CT* const At = static_cast<CT*>(q.At);
     CT* const Bc = static_cast<CT*>(q.Bc);
     CT* const Bt = static_cast<CT*>(q.Bt);
-    const int t = blockIdx.x - q.blk0[kStageConvert];
     const int a_tiles = (q.in + 63) / 64;
     const bool is_a = t < a_tiles;
     const int64_t base = (int64_t)(is_a ? t : t - a_tiles) * 64;
-    const int64_t extent = is_a ? q.in : q.out;
-    // load: element (rank a, index base + j); A is [r][in] (index along a row), B is [out][r]
-    for (int e = threadIdx.x; e < 64 * 32; e += kThreads) {
-        int a, j;
-        if (is_a) { a = e / 64; j = e % 64; }   // consecutive threads: consecutive columns of row a
-        else { j = e / 32; a = e % 32; }        // consecutive threads: consecutive ranks of row j
-        const int64_t idx = base + j;
-        if (a >= r || idx >= extent) continue;
-        const float v = is_a ? q.A[(int64_t)a * q.in + idx] : q.B[idx * r + a];
-        const CT b = (CT)v;
-        tile[j][a] = b;
-        if (is_a) Ac[(int64_t)a * q.in + idx] = b;
-        else Bc[idx * r + a] = b;
+    const int64_t extent = is_a ? q.in : q.out;   // a multiple of 8
+    const int tid = threadIdx.x;
+    // 32 ranks x 8 groups of indices, and 64 indices x 4 groups of ranks (r is a multiple of 8)
+    const int ra = tid >> 3, rj = 8 * (tid & 7), ij = tid >> 2, ia = 8 * (tid & 3);
+    const bool by_rank = ra < r && base + rj < extent, by_index = ia < r && base + ij < extent;
+    const bool ld_ok = is_a ? by_rank : by_index;
+    const int64_t at = is_a ? (int64_t)ra * q.in + base + rj : (base + ij) * r + ia;
+    if (ld_ok) {
+        const float* s = (is_a ? q.A : q.B) + at;
+        const f32x4 x = ldg_f4(s), y = ldg_f4(s + 4);
+        const CT v[8] = {(CT)x[0], (CT)x[1], (CT)x[2], (CT)x[3], (CT)y[0], (CT)y[1], (CT)y[2], (CT)y[3]};
+        store8<CT>((is_a ? Ac : Bc) + at, v);
+        store8<CT>(tile + (is_a ? ra * kConvPitch + rj : ij * kConvPitch + ia), v);
     }
     __syncthreads();
-    // transposed stores: At [in][r] (rows of r ranks), Bt [r][out] (rows of 64 indices)
-    for (int e = threadIdx.x; e < 64 * 32; e += kThreads) {
-        int a, j;
-        if (is_a) { j = e / 32; a = e % 32; }
-        else { a = e / 64; j = e % 64; }
-        const int64_t idx = base + j;
-        if (a >= r || idx >= extent) continue;
-        if (is_a) At[idx * r + a] = tile[j][a];
-        else Bt[(int64_t)a * q.out + idx] = tile[j][a];
+    // transposed stores: At [in][r] (8 ranks of an index), Bt [r][out] (8 indices of a rank)
+    if (is_a ? by_index : by_rank) {
+        CT v[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] = is_a ? tile[(ia + k) * kConvPitch + ij] : tile[(rj + k) * kConvPitch + ra];
+        store8<CT>(is_a ? At + (base + ij) * r + ia : Bt + (int64_t)ra * q.out + base + rj, v);
     }
+}
+template <class CT>
+__global__ __launch_bounds__(kThreads) void group_convert_kernel(const PrepDesc* __restrict__ ds,
+                                                                 const int* __restrict__ block_member, int r) {
+    __shared__ __attribute__((aligned(16))) CT tile[64 * kConvPitch];
+    const PrepDesc& q = ds[block_member[blockIdx.x]];
+    convert_tile<CT>(q, (int)blockIdx.x - q.blk0[kStageConvert], r, tile);
 }
 
 // P^T[a][o] = sum_i A[a][i] W[o][i] for every member, v_mfma_f32_16x16x32_bf16: one block per 256
@@ -1596,41 +1632,62 @@ __device__ __forceinline__ uint4 ldg16(const void* p) {
     return uint4{v.x, v.y, v.z, v.w};
 }
 
-// Every chunk's operands (the raw base chunk, the 64 rows of A^T and the r x 64 slice of A) are
-// loaded cooperatively one chunk ahead, all before the current chunk's stores: the wait for them at
-// the next chunk then does not include those stores (vmcnt counts loads and stores in issue order).
-template <int TYPE>
-__global__ __launch_bounds__(kThreads) void group_merge_kernel(const PrepDesc* __restrict__ ds,
-                                                               const int* __restrict__ block_member, int r, float s) {
+// Every chunk's operands (the raw base chunk and the r x 64 slice of A) are loaded cooperatively one
+// chunk ahead, all before the current chunk's stores: the wait for them at the next chunk then does
+// not include those stores (vmcnt counts loads and stores in issue order). A and B are read as the
+// f32 adapter holds them and rounded here, so the refresh does not wait for the bf16 copies the
+// products read: those are written by conversion blocks behind the merge blocks of the same launch
+// (merge_blocks on). s B A's operand A^T comes from the staged rows of A by transposed LDS reads.
+//
+// msplit > 1: a 64-row block's columns are shared by msplit workgroups; with dora each writes its
+// partial row sums (double) and P (kMergePart floats a block), and the last one to arrive adds them
+// in split order (the rule: merge_splits).
+constexpr int kMergePart = 64 * 32 + 2 * kMergeRows;   // floats: P of 64 rows x 32 ranks, 64 doubles
+__device__ __forceinline__ uint4 pack8_bf16(f32x4 a, f32x4 b) {
+    const bf16 v[8] = {(bf16)a[0], (bf16)a[1], (bf16)a[2], (bf16)a[3], (bf16)b[0], (bf16)b[1], (bf16)b[2], (bf16)b[3]};
+    return __builtin_bit_cast(uint4, v);
+}
+
+template <int TYPE, bool TR, class SRC>   // TR: some member keeps the transposed W_eff too
+__global__ __launch_bounds__(kThreads) void group_merge_kernel(SRC src, int r, float s, int merge_blocks, float* part,
+                                                               int* counters) {
     using MT = MergeType<TYPE>;
     constexpr int RB = 64 * MT::kBytes;                    // raw bytes of one chunk row
     constexpr int RP = RB + 16;                             // LDS pitch of the raw chunk rows
     constexpr int NQ = RB * kMergeRows / 16 / kThreads;     // 16-byte raw loads per thread per chunk (1, 2 or 4)
     constexpr int TPR = RB / 16;                            // threads per raw chunk row
-    constexpr int AP = 80;                                  // LDS pitch of the A^T rows (64 bytes + 16)
     constexpr int CP = 144;                                 // LDS pitch of the A rows (128 bytes + 16)
-    const PrepDesc& q = ds[block_member[blockIdx.x]];
-    if (q.wtype != TYPE) return;   // a member of another element type (its own launch)
     __shared__ __attribute__((aligned(16))) char wraw[kMergeRows * RP];
-    __shared__ __attribute__((aligned(16))) char ats[64 * AP];                  // A^T rows of the chunk [i][a]
     __shared__ __attribute__((aligned(16))) char acs[32 * CP];                  // A rows of the chunk [a][i]
     __shared__ __attribute__((aligned(16))) float wsc[kMergeRows][2];           // Q8_0 scales of the chunk
     __shared__ __attribute__((aligned(16))) bf16 et[kMergeRows][kMergeEP];      // W_eff [o][i] of the chunk
-    __shared__ __attribute__((aligned(16))) bf16 ett[kMergeRows][kMergeEP];     // W_eff^T [i][o] of the chunk
+    __shared__ __attribute__((aligned(16))) bf16 ett[TR ? kMergeRows : 1][kMergeEP];   // W_eff^T [i][o] of the chunk
+    const int bid = blockIdx.x;
+    if (bid >= merge_blocks) {
+        const PrepDesc& q = src.find(kStageConvert, bid);
+        if (q.wtype != TYPE) return;
+        static_assert(sizeof(et) >= 64 * kConvPitch * sizeof(bf16), "conversion tile");
+        convert_tile<bf16>(q, bid - q.blk0[kStageConvert], r, &et[0][0]);
+        return;
+    }
+    const PrepDesc& q = src.find(kStageMerge, bid);
+    if (q.wtype != TYPE) return;   // a member of another element type (its own launch)
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, g = lane >> 4;
     const int64_t in = q.in, out = q.out;
-    const int64_t o0 = (int64_t)(blockIdx.x - q.blk0[kStageMerge]) * kMergeRows;
+    const int msplit = q.msplit, row_blk = (bid - q.blk0[kStageMerge]) / msplit;
+    const int sp = bid - q.blk0[kStageMerge] - row_blk * msplit;
+    const int64_t o0 = (int64_t)row_blk * kMergeRows;
     const bool dora = q.mag != nullptr;
     const bool hi = r > 16;
     const char* wsrc = static_cast<const char*>(q.Wsrc);
-    // this thread's slice of the A^T rows (row tid / 4, bytes 16 (tid % 4)) and of the A rows
-    // (row tid / 8, bytes 16 (tid % 8)); slices past the rank read a valid address and are zeroed
-    const int at_row = tid >> 2, at_b = 16 * (tid & 3), ac_row = tid >> 3, ac_b = 16 * (tid & 7);
-    const bool at_ok = at_b < 2 * r, ac_ok = ac_row < r;
-    const char* at_src = reinterpret_cast<const char*>(q.At) + (int64_t)at_row * r * 2 + (at_ok ? at_b : 0);
-    const char* ac_src = reinterpret_cast<const char*>(q.Ac) + (int64_t)(ac_ok ? ac_row : 0) * in * 2 + ac_b;
+    // this thread's slice of the A rows (row tid / 8, columns 8 (tid % 8) ..); rows past the rank
+    // read a valid address and are zeroed
+    const int ac_row = tid >> 3, ac_b = 16 * (tid & 7);
+    const bool ac_ok = ac_row < r;
+    const float* ac_src = q.A + (int64_t)(ac_ok ? ac_row : 0) * in + 8 * (tid & 7);
     struct Stage {
-        uint4 w[NQ], at, ac;
+        uint4 w[NQ];
+        f32x4 a0, a1;
         uint32_t sc;   // Q8_0: the chunk row's two f16 block scales (threads < 64)
     } st;
     auto load = [&](int64_t i0) {
@@ -1640,8 +1697,8 @@ __global__ __launch_bounds__(kThreads) void group_merge_kernel(const PrepDesc* _
             const int64_t o = min(o0 + row, out - 1);   // rows past out are never stored
             st.w[k] = ldg16(wsrc + (o * in + i0) * MT::kBytes + (e % TPR) * 16);
         }
-        st.at = ldg16(at_src + i0 * r * 2);
-        st.ac = ldg16(ac_src + i0 * 2);
+        st.a0 = ldg_f4(ac_src + i0);
+        st.a1 = ldg_f4(ac_src + i0 + 4);
         if constexpr (TYPE == SA3K_TYPE_Q8_0) {
             const int64_t o = min(o0 + (tid & 63), out - 1);
             st.sc = *(__attribute__((address_space(1))) const uint32_t*)(static_cast<const uint16_t*>(q.Wsc) + o * (in / 32) + i0 / 32);
@@ -1649,29 +1706,30 @@ __global__ __launch_bounds__(kThreads) void group_merge_kernel(const PrepDesc* _
     };
     // delta's A operand: the rank entries 8g.. of B row o (this wave's 16 rows), loop-invariant
     const int64_t ob = min(o0 + 16 * wave + l16, out - 1);
+    const float* b_src = q.B + ob * r + (8 * g < r ? 8 * g : 0);
     const bf16x8 zero8 = {};
-    const bf16x8 bop = 8 * g < r ? __builtin_bit_cast(bf16x8, ldg16(static_cast<const bf16*>(q.Bc) + ob * r + (8 * g < r ? 8 * g : 0))) : zero8;
+    const bf16x8 bop = 8 * g < r ? __builtin_bit_cast(bf16x8, pack8_bf16(ldg_f4(b_src), ldg_f4(b_src + 4))) : zero8;
     double nacc[4] = {0.0, 0.0, 0.0, 0.0};   // rows 16 wave + 4g + v, this lane's columns
     f32x4 p0 = {0.f, 0.f, 0.f, 0.f}, p1 = {0.f, 0.f, 0.f, 0.f};
     const uint32_t wbytes = (uint32_t)(out * in * 2);   // < 2^31 (checked when the group is built)
     const __amdgpu_buffer_rsrc_t rs_m = __builtin_amdgcn_make_buffer_rsrc(q.Wm, (short)0, (int)wbytes, 0x00020000);
-    const __amdgpu_buffer_rsrc_t rs_mt = __builtin_amdgcn_make_buffer_rsrc(q.Wmt, (short)0, (int)wbytes, 0x00020000);
-    load(0);
+    [[maybe_unused]] const __amdgpu_buffer_rsrc_t rs_mt = __builtin_amdgcn_make_buffer_rsrc(q.Wmt, (short)0, (int)wbytes, 0x00020000);
+    const int cps = (int)((in / 64 + msplit - 1) / msplit), c0 = sp * cps, c1 = min(c0 + cps, (int)(in / 64));
+    load((int64_t)c0 * 64);
     // the first chunk landed: the loop head's wait then only reflects the loop body's issue order
     // (a scheduler-reordered prologue would otherwise force a full wait there every chunk)
     __builtin_amdgcn_s_waitcnt(0x3F70);   // vmcnt(0)
-    const int nc = (int)(in / 64);
-    for (int c = 0; c < nc; ++c) {
+    for (int c = c0; c < c1; ++c) {
         const int64_t i0 = (int64_t)c * 64;
 #pragma unroll
         for (int k = 0; k < NQ; ++k) {
             const int e = tid + k * kThreads;
             *reinterpret_cast<uint4*>(wraw + (e / TPR) * RP + (e % TPR) * 16) = st.w[k];
         }
-        {   // slices past the rank are zeroed arithmetically (no branch: see the stores below)
-            const uint32_t ma = at_ok ? ~0u : 0u, mc = ac_ok ? ~0u : 0u;
-            *reinterpret_cast<uint4*>(ats + at_row * AP + at_b) = uint4{st.at.x & ma, st.at.y & ma, st.at.z & ma, st.at.w & ma};
-            *reinterpret_cast<uint4*>(acs + ac_row * CP + ac_b) = uint4{st.ac.x & mc, st.ac.y & mc, st.ac.z & mc, st.ac.w & mc};
+        {   // rows past the rank are zeroed arithmetically (no branch: see the stores below)
+            const uint32_t mc = ac_ok ? ~0u : 0u;
+            const uint4 a = pack8_bf16(st.a0, st.a1);
+            *reinterpret_cast<uint4*>(acs + ac_row * CP + ac_b) = uint4{a.x & mc, a.y & mc, a.z & mc, a.w & mc};
         }
         if constexpr (TYPE == SA3K_TYPE_Q8_0) {
             if (tid < kMergeRows) {
@@ -1679,10 +1737,10 @@ __global__ __launch_bounds__(kThreads) void group_merge_kernel(const PrepDesc* _
                 wsc[tid][1] = (float)__builtin_bit_cast(_Float16, (uint16_t)(st.sc >> 16));
             }
         }
-        if (c + 1 < nc) load(i0 + 64);   // the next chunk in flight
+        if (c + 1 < c1) load(i0 + 64);   // the next chunk in flight
         __syncthreads();   // the chunk is staged; the previous chunk's W_eff tiles are consumed
-        // The P product's A operands (this chunk's A rows) are read before the second barrier: a
-        // wave past that barrier may already be writing the next chunk's A rows into acs.
+        // The A operands of both products are read before the second barrier: a wave past that
+        // barrier may already be writing the next chunk's A rows into acs.
         bf16x8 pa[2][2] = {};
         if (dora) {
 #pragma unroll
@@ -1694,7 +1752,8 @@ __global__ __launch_bounds__(kThreads) void group_merge_kernel(const PrepDesc* _
         // W_eff at (row 16 wave + 4g + v, column 16j + l16)
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const bf16x8 atj = *reinterpret_cast<const bf16x8*>(ats + (16 * j + l16) * AP + 16 * g);
+            // lane: column 16j + l16, ranks 8g .. 8g + 7 (rows of acs), two transposed reads of four
+            const bf16x8 atj = cat44(tn_ld_tr(acs, CP, 8 * g, 16 * j, lane), tn_ld_tr(acs, CP, 8 * g + 4, 16 * j, lane));
             const f32x4 dl = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bop, atj, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
             bf16 e4[4];
 #pragma unroll
@@ -1708,7 +1767,8 @@ __global__ __launch_bounds__(kThreads) void group_merge_kernel(const PrepDesc* _
                 et[row][col] = e;
                 if (dora) nacc[v] += (double)sd * (2.0 * (double)w + (double)sd);
             }
-            if (q.Wmt) *reinterpret_cast<uint2*>(&ett[16 * j + l16][16 * wave + 4 * g]) = __builtin_bit_cast(uint2, e4);
+            if constexpr (TR)
+                if (q.Wmt) *reinterpret_cast<uint2*>(&ett[16 * j + l16][16 * wave + 4 * g]) = __builtin_bit_cast(uint2, e4);
         }
         __syncthreads();   // et, ett staged
         if (dora) {   // P += W_eff A^T over the chunk (rows 16 wave + l16 of W_eff as the A operand)
@@ -1724,14 +1784,16 @@ __global__ __launch_bounds__(kThreads) void group_merge_kernel(const PrepDesc* _
             // so no branch makes the wait for the next chunk's loads also wait for these stores.
             const int lr = tid >> 2, lc = 16 * (tid & 3);
             const uint4* fr = reinterpret_cast<const uint4*>(&et[lr][lc]);
-            const uint4* tr = reinterpret_cast<const uint4*>(&ett[lr][lc]);
             const uint32_t fo = o0 + lr < out ? (uint32_t)(((o0 + lr) * in + i0 + lc) * 2) : 0xFFFFFFE0u;
-            const uint32_t to = o0 + lc < out ? (uint32_t)(((i0 + lr) * out + o0 + lc) * 2) : 0xFFFFFFE0u;
             __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4g, fr[0]), rs_m, fo, 0, 0);
             __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4g, fr[1]), rs_m, fo + 16, 0, 0);
-            if (q.Wmt) {
-                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4g, tr[0]), rs_mt, to, 0, 0);
-                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4g, tr[1]), rs_mt, to + 16, 0, 0);
+            if constexpr (TR) {
+                if (q.Wmt) {
+                    const uint4* tr = reinterpret_cast<const uint4*>(&ett[lr][lc]);
+                    const uint32_t to = o0 + lc < out ? (uint32_t)(((i0 + lr) * out + o0 + lc) * 2) : 0xFFFFFFE0u;
+                    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4g, tr[0]), rs_mt, to, 0, 0);
+                    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4g, tr[1]), rs_mt, to + 16, 0, 0);
+                }
             }
         }
     }
@@ -1740,6 +1802,53 @@ __global__ __launch_bounds__(kThreads) void group_merge_kernel(const PrepDesc* _
 #pragma unroll
     for (int v = 0; v < 4; ++v)
         for (int off = 1; off < 16; off <<= 1) nacc[v] += __shfl_xor(nacc[v], off, 16);
+    if (msplit > 1) {
+        // 16 bytes a lane, consecutive lanes consecutive: each wave writes whole lines (device-coherent)
+        float* mine = part + (int64_t)bid * kMergePart;
+        const __amdgpu_buffer_rsrc_t rs_w = __builtin_amdgcn_make_buffer_rsrc(mine, (short)0, kMergePart * 4, 0x00020000);
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4g, p0), rs_w, tid * 16, 0, kSc1);
+        if (hi) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4g, p1), rs_w, 4096 + tid * 16, 0, kSc1);
+        double* md = reinterpret_cast<double*>(mine + 64 * 32);
+        if (l16 == 0) {
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                __hip_atomic_store(md + 16 * wave + 4 * g + v, nacc[v], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        __shared__ int s_last;
+        __shared__ double rowsum[kMergeRows];
+        const int b0 = bid - sp;
+        if (!arrive_last(&counters[b0], msplit, &s_last)) return;
+        const float* all = part + (int64_t)b0 * kMergePart;
+        const __amdgpu_buffer_rsrc_t rs_p = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<float*>(all), (short)0, (int)(msplit * kMergePart * 4), 0x00020000);
+        // the sums in split order from zero, eight splits' loads in flight (past the last split: the
+        // descriptor's end, zeros that are not added)
+        p0 = p1 = f32x4{0.f, 0.f, 0.f, 0.f};
+        double rs = 0.0;
+        for (int z0 = 0; z0 < msplit; z0 += 8) {
+            f32x4 v0[8], v1[8];
+            double dv[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const uint32_t o = (uint32_t)((z0 + k) * kMergePart * 4 + tid * 16);
+                v0[k] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs_p, o, 0, kSc1));
+                if (hi) v1[k] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs_p, o + 4096, 0, kSc1));
+                dv[k] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(
+                                                       rs_p, (z0 + k) * kMergePart * 4 + 8192 + (tid & 63) * 8, 0, kSc1));
+            }
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                if (z0 + k < msplit) {
+                    p0 += v0[k];
+                    if (hi) p1 += v1[k];
+                    rs += dv[k];
+                }
+        }
+        if (tid < kMergeRows) rowsum[tid] = rs;
+        __syncthreads();
+#pragma unroll
+        for (int v = 0; v < 4; ++v) nacc[v] = rowsum[16 * wave + 4 * g + v];
+    }
     const int64_t orow = o0 + 16 * wave + 4 * g;
     if (orow >= out) return;   // out is a multiple of 16: a 4-row group is wholly in or out
     if (l16 == 0) {
@@ -1787,12 +1896,138 @@ void weight_fwd_operand(const sa3k_weight* W, GemmDesc& g) {
     g.ldbs = wo.lds;
 }
 
+namespace {
+
+// The descriptor of one member; merged: W_eff's buffers are made here (on the linear's first
+// merged refresh). The dX product reads W_eff as it lies ([out][in] as a [K][N] operand) unless the
+// transposed copy is asked for (option merge_kn 0).
+PrepDesc prep_desc(sa3k_ctx* ctx, sa3k_lin* L, const float* A, const float* B, const float* mag, const float* bnsq,
+                   bool merged) {
+    const int64_t in = L->W->in, out = L->W->out;
+    PrepDesc q{};
+    q.A = A; q.B = B; q.mag = mag; q.bnsq = bnsq;
+    q.Ac = L->Ac; q.At = L->At; q.Bc = L->Bc; q.Bt = L->Bt;
+    q.W = static_cast<const bf16*>(L->W->wb);
+    q.Pt = L->Pt; q.G = L->G; q.BG = L->BG; q.nsq = L->nsq; q.d = L->d;
+    q.in = (int)in; q.out = (int)out;
+    q.Wsrc = L->W->w; q.Wsc = L->W->ws; q.wtype = L->W->type;
+    q.msplit = 1;
+    if (merged) {
+        if (!L->Wm) L->Wm = dev_alloc<bf16>(in * out);
+        if (!ctx->merge_kn && !L->Wmt) L->Wmt = dev_alloc<bf16>(in * out);
+        if (ctx->merge_kn && L->Wmt) {
+            SA3K_HIP(hipStreamSynchronize(ctx->stream));
+            SA3K_HIP(hipFree(L->Wmt));
+            L->Wmt = nullptr;
+        }
+        q.Wm = static_cast<bf16*>(L->Wm);
+        q.Wmt = static_cast<bf16*>(L->Wmt);
+    }
+    return q;
+}
+
+// Column splits of a member's 64-row blocks, by the 64 x 64 chunks of the whole refresh: a workgroup
+// walks its chunks one after another, about 1.3 us each (a memory round trip and two barriers), so
+// below a chip full of workgroups (four per CU) the time is that walk's length. A group that fills
+// the chip by its rows alone is not split; at least kMergeMinChunks chunks stay with a workgroup.
+// Measured on MI355X, whole refresh unsplit -> split, us: a 1536-wide block's seven linears (one
+// launch) dora r32 117 -> 68, lora r16 111 -> 56; one linear, dora r32: 1536 x 6144 Q8_0 38 -> 21,
+// 1536 x 9216 f16 34 -> 23, 6144 x 1536 f16 107 -> 20. Slots 768 / 2048 and minima of 6 / 8 chunks
+// were within 5% or slower.
+constexpr int kMergeSlots = 1024, kMergeMinChunks = 4;
+int merge_splits(int64_t chunks, int64_t in) {
+    const int64_t nc = in / 64, per = std::max<int64_t>(kMergeMinChunks, ceil_div(chunks, kMergeSlots));
+    const int64_t s = ceil_div(nc, per);
+    return (int)ceil_div(nc, ceil_div(nc, s));   // no split without chunks
+}
+
+// one launch per stored element type present (blocks of other members exit at once)
+template <class SRC>
+void launch_merge(sa3k_ctx* ctx, const SRC& src, sa3k_lin* const* lins, int n, int blocks, int merge_blocks, int r,
+                  float s, float* part) {
+    double bytes = 0.0;
+    bool has[4] = {false, false, false, false}, tr = false;
+    for (int i = 0; i < n; ++i) {
+        const sa3k_weight* W = lins[i]->W;
+        bytes += (double)W->in * (double)W->out * (type_size(W->type) + 4.0);
+        has[W->type == SA3K_TYPE_F32 ? 0 : W->type == SA3K_TYPE_F16 ? 1 : W->type == SA3K_TYPE_BF16 ? 2 : 3] = true;
+        tr = tr || lins[i]->Wmt;
+    }
+    SA3K_REQUIRE(!part || stream_counters(ctx), "column splits on a stream without arrival counters");
+    KernelScope ks(ctx, "group_merge", bytes);
+    using K = void (*)(SRC, int, float, int, float*, int*);
+    const K kern[2][4] = {{group_merge_kernel<SA3K_TYPE_F32, false, SRC>, group_merge_kernel<SA3K_TYPE_F16, false, SRC>,
+                           group_merge_kernel<SA3K_TYPE_BF16, false, SRC>, group_merge_kernel<SA3K_TYPE_Q8_0, false, SRC>},
+                          {group_merge_kernel<SA3K_TYPE_F32, true, SRC>, group_merge_kernel<SA3K_TYPE_F16, true, SRC>,
+                           group_merge_kernel<SA3K_TYPE_BF16, true, SRC>, group_merge_kernel<SA3K_TYPE_Q8_0, true, SRC>}};
+    for (int t = 0; t < 4; ++t) {
+        if (!has[t]) continue;
+        kern[tr][t]<<<(unsigned)blocks, kThreads, 0, ctx->stream>>>(src, r, s, merge_blocks, part, stream_counters(ctx));
+        SA3K_LAUNCHED();
+    }
+}
+
+}  // namespace
+
+bool lin_prepare_merged(sa3k_ctx* ctx, sa3k_lin* const* lins, int n, const float* const* A, const float* const* B,
+                        const float* const* mag, const float* const* bnsq, float scale, int dora) {
+    if (n < 1 || n > kInlineMax || !ctx->lin_merge) return false;
+    for (int i = 0; i < n; ++i) {
+        const sa3k_lin* L = lins[i];
+        if (L->prec != SA3K_PREC_BF16 || L->rank <= 0 || L->rank != lins[0]->rank || L->W->out % 16 != 0) return false;
+    }
+    for (int i = 0; i < n; ++i) {
+        SA3K_REQUIRE(A[i] && B[i] && (!dora || (mag[i] && bnsq[i])), "missing adapter pointer");
+        SA3K_REQUIRE(lins[i]->W->out * lins[i]->W->in * 2 < ((int64_t)1 << 31), "group member weight above 2 GiB");
+    }
+    std::vector<sa3k_lin*> order(lins, lins + n);   // the longest members first, as in a group
+    std::vector<int> idx(n);
+    for (int i = 0; i < n; ++i) idx[i] = i;
+    std::stable_sort(idx.begin(), idx.end(), [&](int a, int b) { return lins[a]->W->in > lins[b]->W->in; });
+    PrepInline src{};
+    src.n = n;
+    int64_t chunks = 0;
+    for (int i = 0; i < n; ++i) chunks += ceil_div(lins[i]->W->out, kMergeRows) * (lins[i]->W->in / 64);
+    int blocks = 0;
+    bool split = false;
+    for (int k = 0; k < n; ++k) {
+        const int i = idx[k];
+        order[k] = lins[i];
+        PrepDesc& q = src.ds[k];
+        q = prep_desc(ctx, lins[i], A[i], B[i], dora ? mag[i] : nullptr, dora ? bnsq[i] : nullptr, true);
+        q.msplit = merge_splits(chunks, q.in);
+        if (dora && !stream_counters(ctx)) q.msplit = 1;
+        split = split || q.msplit > 1;
+        q.blk0[kStageMerge] = blocks;
+        blocks += (int)ceil_div(q.out, kMergeRows) * q.msplit;
+    }
+    const int merge_blocks = blocks;
+    if (split && dora) SA3K_REQUIRE(merge_blocks <= kMaxFixupTiles, "column splits need an arrival counter per block");
+    for (int k = 0; k < n; ++k) {
+        src.ds[k].blk0[kStageConvert] = blocks;
+        blocks += (int)(ceil_div(src.ds[k].in, 64) + ceil_div(src.ds[k].out, 64));
+    }
+    float* part = split && dora ? reduce_workspace(ctx, (size_t)merge_blocks * kMergePart * sizeof(float)) : nullptr;
+    for (int i = 0; i < n; ++i) {   // the per-linear state sa3k_lin_prepare sets
+        sa3k_lin* L = lins[i];
+        L->s = scale;
+        L->dora = dora ? 1 : 0;
+        L->B = B[i];
+        L->mag = dora ? mag[i] : nullptr;
+        L->merged = 1;
+    }
+    launch_merge(ctx, src, order.data(), n, blocks, merge_blocks, lins[0]->rank, scale, part);
+    return true;
+}
+
 struct LinGroup {
     std::vector<sa3k_lin*> lins;
     std::vector<const float*> B, mag;
     PrepDesc* dev = nullptr;
     int* block_member[kStages] = {};   // per stage: the member of every block
     int blocks[kStages] = {};
+    float* part = nullptr;             // merged: partial row sums and P of the column splits
+    int merge_blocks = 0, split = 0;   // merged: blocks before the conversion's; any member split
     int n = 0, r = 0, dora = 0, merged = 0;
     int f32 = 0;   // members compute in f32: f32 copies, P on the VALU from the stored base
     float s = 1.0f;
@@ -1801,6 +2036,7 @@ struct LinGroup {
 void lin_group_free(LinGroup* g) {
     if (!g) return;
     if (g->dev) (void)hipFree(g->dev);
+    if (g->part) (void)hipFree(g->part);
     for (int* b : g->block_member)
         if (b) (void)hipFree(b);
     delete g;
@@ -1834,26 +2070,8 @@ LinGroup* lin_group_create(sa3k_ctx* ctx, sa3k_lin* const* lins, int n, const fl
             const int64_t in = L->W->in, out = L->W->out;
             SA3K_REQUIRE(out % 64 == 0 || out % 16 == 0, "group output dimension must be a multiple of 16");
             SA3K_REQUIRE((int64_t)out * in * 2 < ((int64_t)1 << 31), "group member weight above 2 GiB");
+            h[i] = prep_desc(ctx, L, A[i], B[i], dora ? mag[i] : nullptr, dora ? bnsq[i] : nullptr, g->merged != 0);
             PrepDesc& q = h[i];
-            q.A = A[i]; q.B = B[i]; q.mag = dora ? mag[i] : nullptr; q.bnsq = dora ? bnsq[i] : nullptr;
-            q.Ac = L->Ac; q.At = L->At; q.Bc = L->Bc; q.Bt = L->Bt;
-            q.W = static_cast<const bf16*>(L->W->wb);
-            q.Pt = L->Pt; q.G = L->G; q.BG = L->BG; q.nsq = L->nsq; q.d = L->d;
-            q.in = (int)in; q.out = (int)out;
-            q.Wsrc = L->W->w; q.Wsc = L->W->ws; q.wtype = L->W->type;
-            q.Wm = q.Wmt = nullptr;
-            if (g->merged) {
-                // the dX product reads W_eff as it lies ([out][in] as a [K][N] operand) unless the
-                // transposed copy is asked for (option merge_kn 0)
-                if (!L->Wm) L->Wm = dev_alloc<bf16>(in * out);
-                if (!ctx->merge_kn && !L->Wmt) L->Wmt = dev_alloc<bf16>(in * out);
-                if (ctx->merge_kn && L->Wmt) {
-                    SA3K_HIP(hipFree(L->Wmt));
-                    L->Wmt = nullptr;
-                }
-                q.Wm = static_cast<bf16*>(L->Wm);
-                q.Wmt = static_cast<bf16*>(L->Wmt);
-            }
             const int64_t per_stage[kStages] = {ceil_div(in, 64) + ceil_div(out, 64),
                                                 ceil_div(out, g->f32 ? kPtRowsF32 : kPtRows),
                                                 ceil_div(in, kGramCols), ceil_div(out, kTermRows),
@@ -1871,9 +2089,20 @@ LinGroup* lin_group_create(sa3k_ctx* ctx, sa3k_lin* const* lins, int n, const fl
             std::vector<int> order(n);
             for (int i = 0; i < n; ++i) order[i] = i;
             std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return h[a].in > h[b].in; });
+            int64_t chunks = 0;
+            for (const PrepDesc& q : h) chunks += ceil_div(q.out, kMergeRows) * (q.in / 64);
             for (int i : order) {
+                h[i].msplit = merge_splits(chunks, h[i].in);
+                g->split |= h[i].msplit > 1;
                 h[i].blk0[kStageMerge] = (int)bm[kStageMerge].size();
-                bm[kStageMerge].insert(bm[kStageMerge].end(), (size_t)ceil_div(h[i].out, kMergeRows), i);
+                bm[kStageMerge].insert(bm[kStageMerge].end(), (size_t)(ceil_div(h[i].out, kMergeRows) * h[i].msplit), i);
+            }
+            g->merge_blocks = (int)bm[kStageMerge].size();
+            if (g->merged) {   // the conversion blocks ride behind the merge blocks of the same launch
+                SA3K_REQUIRE(!g->split || g->merge_blocks <= kMaxFixupTiles, "column splits need an arrival counter per block");
+                if (g->split && g->dora) g->part = dev_alloc<float>((int64_t)g->merge_blocks * kMergePart);
+                for (PrepDesc& q : h) q.blk0[kStageConvert] += g->merge_blocks;
+                bm[kStageMerge].insert(bm[kStageMerge].end(), bm[kStageConvert].begin(), bm[kStageConvert].end());
             }
         }
         SA3K_HIP(hipMalloc(&g->dev, sizeof(PrepDesc) * n));
@@ -1904,30 +2133,17 @@ void lin_group_prepare(sa3k_ctx* ctx, LinGroup* g) {
         L->mag = g->mag[i];
         L->merged = g->merged;
     }
+    if (g->merged) {
+        launch_merge(ctx, PrepTable{g->dev, g->block_member[kStageMerge]}, g->lins.data(), g->n,
+                     g->blocks[kStageMerge], g->merge_blocks, g->r, g->s, g->part);
+        return;
+    }
     {
         KernelScope ks(ctx, "group_convert");
         auto* kern = g->f32 ? group_convert_kernel<float> : group_convert_kernel<bf16>;
         kern<<<(unsigned)g->blocks[kStageConvert], kThreads, 0, ctx->stream>>>(g->dev, g->block_member[kStageConvert],
                                                                             g->r);
         SA3K_LAUNCHED();
-    }
-    if (g->merged) {
-        double bytes = 0.0;
-        for (sa3k_lin* L : g->lins) bytes += (double)L->W->in * (double)L->W->out * (type_size(L->W->type) + 4.0);
-        KernelScope ks(ctx, "group_merge", bytes);
-        // one launch per element type present (blocks of other members exit at once)
-        bool has[4] = {false, false, false, false};
-        for (sa3k_lin* L : g->lins) has[L->W->type == SA3K_TYPE_F32 ? 0 : L->W->type == SA3K_TYPE_F16 ? 1 : L->W->type == SA3K_TYPE_BF16 ? 2 : 3] = true;
-        void (*kern[4])(const PrepDesc*, const int*, int, float) = {
-            group_merge_kernel<SA3K_TYPE_F32>, group_merge_kernel<SA3K_TYPE_F16>, group_merge_kernel<SA3K_TYPE_BF16>,
-            group_merge_kernel<SA3K_TYPE_Q8_0>};
-        for (int t = 0; t < 4; ++t) {
-            if (!has[t]) continue;
-            kern[t]<<<(unsigned)g->blocks[kStageMerge], kThreads, 0, ctx->stream>>>(g->dev, g->block_member[kStageMerge],
-                                                                                 g->r, g->s);
-            SA3K_LAUNCHED();
-        }
-        return;
     }
     if (!g->dora) return;
     {
@@ -1996,7 +2212,7 @@ LinStack* lin_stack_create(sa3k_ctx* ctx, sa3k_lin* const* lins, int n) {
     for (int i = 0; i < n; ++i) {
         const sa3k_lin* L = lins[i];
         if (L->prec != SA3K_PREC_BF16 || L->rank != L0->rank || L0->rank <= 0 || L->W->in != L0->W->in ||
-            L->W->out != L0->W->out || L->max_tokens != L0->max_tokens || L->ext != 0 || L->Wm || L->solo)
+            L->W->out != L0->W->out || L->max_tokens != L0->max_tokens || L->ext != 0 || L->Wm)
             return nullptr;
     }
     if (L0->W->out % 8 != 0 || (int64_t)n * L0->W->out * L0->W->in * 2 >= ((int64_t)1 << 31)) return nullptr;
@@ -2245,21 +2461,7 @@ SA3K_API int sa3k_lin_prepare(sa3k_ctx* ctx, sa3k_lin* L, const float* A, const 
         const bool bf = L->prec == SA3K_PREC_BF16;
         L->merged = 0;
         if (bf && ctx->lin_merge && out % 16 == 0) {
-            // the merged refresh through a one-member group, rebuilt when the adapter changes
-            const float* key[4] = {A, B, dora ? magnitude : nullptr, dora ? base_norm_sq : nullptr};
-            if (!L->solo || !std::equal(key, key + 4, L->solo_key) || L->solo_s != scale || L->solo_dora != dora) {
-                if (L->solo) {
-                    SA3K_HIP(hipStreamSynchronize(ctx->stream));
-                    lin_group_free(L->solo);
-                    L->solo = nullptr;
-                }
-                sa3k_lin* one = L;
-                L->solo = lin_group_create(ctx, &one, 1, &key[0], &key[1], &key[2], &key[3], scale, dora);
-                std::copy(key, key + 4, L->solo_key);
-                L->solo_s = scale;
-                L->solo_dora = dora;
-            }
-            lin_group_prepare(ctx, L->solo);
+            lin_prepare_merged(ctx, &L, 1, &A, &B, &magnitude, &base_norm_sq, scale, dora);
             return;
         }
         KernelScope ks(ctx, "lin_prepare");

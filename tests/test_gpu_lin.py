@@ -220,6 +220,34 @@ def test_merged_refresh_terms(ctx, wt, r):
         assert rel_err(got[k], seg[k]) < 1e-2, k
 
 
+@pytest.mark.parametrize("in_,out_,r", [(6144, 64, 32), (1536, 128, 8), (320, 192, 24), (256, 64, 16), (64, 64, 32)])
+@pytest.mark.parametrize("dora", [True, False])
+def test_merged_refresh_column_splits(ctx, in_, out_, r, dora):
+    """The refresh of one linear with its 64-row blocks' columns over several workgroups (24 of them,
+    6 of 4 chunks, 2 of 3 and 2 chunks, and none), from an adapter that starts 4
+    bytes off a 16-byte boundary: against the oracle, and bit for bit the same twice."""
+    N = 33
+    X, dY, W, A, B = make_inputs(17, N, in_, out_, r, w_sd=0.05, b_sd=0.05)
+    Wh = W.astype(np.float16)
+    Wdec = Wh.astype(np.float32)
+    mag = (oracle.row_norms(Wdec) * 0.9 + 0.01).astype(np.float32)
+    ref = run_oracle(X, dY, Wdec, A, B, 0.75, dora, mag)
+    one = run_gpu(ctx, X, dY, Wh, sa3k.TYPE_F16, A, B, 0.75, dora, mag, sa3k.PREC_BF16)
+    w = ctx.weight(Wh, sa3k.TYPE_F16)
+    lin = ctx.lin(w, r, sa3k.PREC_BF16, N)
+    flat = ctx.upload(np.concatenate([[0.0], A.ravel(), B.ravel()]).astype(np.float32))
+    odd = [sa3k.DeviceArray(ctx, flat.ptr + 4 * o, shape, np.float32, owner=False)
+           for o, shape in ((1, A.shape), (1 + A.size, B.shape))]
+    lin.prepare(*odd, 0.75, dora, ctx.upload(mag) if dora else None, w.row_norm_sq(1e-12) if dora else None)
+    Y = ctx.empty((N, out_))
+    lin.forward(ctx.upload(X), N, Y)
+    assert np.array_equal(Y.numpy(), one["Y"])
+    lin.destroy()
+    w.destroy()
+    for k in ("Y", "dX", "dA", "dB") + (("dm",) if dora else ()):   # bf16 operands, as above
+        assert rel_err(one[k], ref[k]) < 2e-2 and cosine(one[k], ref[k]) >= 0.9999, k
+
+
 @pytest.mark.parametrize("kn", [0, 1])
 @pytest.mark.parametrize("cols", [0, 1, 2, 3])
 def test_rank_products_as_extra_columns(ctx, cols, kn):
