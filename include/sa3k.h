@@ -102,10 +102,11 @@ SA3K_API int sa3k_vec_add(sa3k_ctx* ctx, float* dst_dev, const float* src_dev, i
  *                 (and 16-wave 256 x 256 tiles where those are taken) and 128 x 128 for f32;
  *                 1: 128 x 128; 4: 128 x 256 and 256 x 256 of 8 waves (3 / 2 stages);
  *                 7: 128 x 256 of 8 waves (2 stages)
- *   "gemm_small"  DMA kernel tile configuration for GEMMs whose 128x128 grid cannot fill the chip
- *                 (default 4: bf16 128x128 tiles of eight waves at any K, f32 and decoded B 64x128
- *                 below K 2048 / 4096; 2: 64x128 tiles below those K; 0: the default tile, split
- *                 over K)
+ *   "gemm_small"  default 4: the tile and split count of a bf16 product with both operands in bf16
+ *                 are those with the least estimated time (with gemm_big 3, gemm_cfg 0 or 4 and
+ *                 no forced split), f32 products take the tiles that load the CUs most evenly;
+ *                 2: 64x128 tiles below K 4096 (f32: 2048) where the 128x128 grid cannot fill the
+ *                 chip; 0: there the default tile, split over K
  *   "gemm_nt_store" 1: GEMM outputs are written with non-temporal stores (default 1)
  *   "gemm_skinny" 1: bf16 products with at most 32 output columns and a plain epilogue (the rank
  *                 products s X A^T and s dU B) run on a kernel that splits K across the waves of

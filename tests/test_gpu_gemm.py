@@ -155,6 +155,36 @@ def test_skinny_gemm(ctx, M, N, K):
     assert max_rel_err(got, tiled) < 1e-5
 
 
+@pytest.mark.parametrize("K", [64, 128, 256, 448, 576, 1600])
+@pytest.mark.parametrize("M,N", [(1, 72), (31, 200), (33, 1536), (65, 1000), (343, 1536), (343, 4608), (279, 12288),
+                                 (700, 328)])
+def test_planned_tiles(ctx, M, N, K):
+    # the tiles and splits chosen for small and ragged products, over K loops shorter and longer than
+    # the tiles' rings: f32 accumulation error only (K products of unit and 0.02 scale: well below
+    # 1e-5 of the 2-norm), bit-identical on a repeat, bias and column factors applied
+    r = rng(M * 5 + N * 3 + K)
+    A = r.normal(0, 1, (M, K)).astype(np.float32)
+    W = r.normal(0, 0.02, (N, K)).astype(np.float32)
+    bias = r.normal(0, 1, N).astype(np.float32)
+    cs = r.uniform(0.5, 1.5, N).astype(np.float32)
+    args = (bf16_bits(A), bf16_bits(W), M, N, K, sa3k.PREC_BF16, sa3k.TYPE_BF16, sa3k.TYPE_BF16)
+    got = run(ctx, *args, bias=bias, colscale=cs)
+    again = run(ctx, *args, bias=bias, colscale=cs)
+    ref = (bf16_round(A).astype(np.float64) @ bf16_round(W).astype(np.float64).T) * cs + bias
+    assert np.array_equal(got, again), "not deterministic"
+    assert rel_err(got, ref) < 1e-5
+
+
+@pytest.mark.parametrize("M,N,K", [(2048, 1536, 512), (1990, 1500, 96), (4000, 2048, 64)])
+def test_f32_tiles(ctx, M, N, K):
+    # f32 products whose 64 x 128 tiles fill the CUs unevenly (64 x 64 tiles there) and evenly
+    r = rng(M + N + K)
+    A = r.normal(0, 1, (M, K)).astype(np.float32)
+    W = r.normal(0, 0.02, (N, K)).astype(np.float32)
+    got = run(ctx, A, W, M, N, K, sa3k.PREC_F32, sa3k.TYPE_F32, sa3k.TYPE_F32)
+    assert rel_err(got, A.astype(np.float64) @ W.astype(np.float64).T) < 1e-6 * max(1.0, (K / 64) ** 0.5)
+
+
 @pytest.mark.parametrize("M,N,K", [(2176, 12288, 1536), (2176, 6144, 1536), (300, 640, 256), (520, 1000, 192),
                                    (2176, 1536, 6144)])
 def test_big_tile_gemm(ctx, M, N, K):

@@ -303,6 +303,22 @@ def test_tile_configurations(ctx, opts):
             assert rel_err(got[k], ref[k]) < 2e-2 and cosine(got[k], ref[k]) >= 0.9999, (N, in_, out_, k)
 
 
+@pytest.mark.parametrize("N", [1, 37, 100, 343])
+def test_dora_odd_tokens(ctx, N):
+    """Token counts that are no multiple of 8: the dX product's extra DoRA rows start on the next
+    8-row boundary of the tile grid, and the rows between are never stored. Small and split shapes;
+    the bar is the bf16 one of the other tests against the oracle."""
+    for in_, out_, r in ((192, 320, 16), (1536, 1536, 32), (256, 6144, 8)):
+        X, dY, W, A, B = make_inputs(43, N, in_, out_, r)
+        Wh = W.astype(np.float16)
+        Wdec = Wh.astype(np.float32)
+        mag = (oracle.row_norms(Wdec) * 0.97).astype(np.float32)
+        got = run_gpu(ctx, X, dY, Wh, sa3k.TYPE_F16, A, B, 1.25, True, mag, sa3k.PREC_BF16)
+        ref = run_oracle(X, dY, Wdec, A, B, 1.25, True, mag)
+        for k in ("Y", "dX", "dA", "dB", "dm"):
+            assert rel_err(got[k], ref[k]) < 2e-2 and cosine(got[k], ref[k]) >= 0.9999, (N, in_, out_, k)
+
+
 @pytest.mark.parametrize("big", [0, 1, 2])
 def test_dx_k_major_operand(ctx, big):
     """Merged linears' dX product reads W + s B A in its stored [out][in] layout as a K-major B
