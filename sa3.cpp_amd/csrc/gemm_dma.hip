@@ -382,30 +382,32 @@ bool plain_ok(const DmaParams& p) {
 // 279 x 12288 on 64 x 256 or 128 x 256 20, 128 x 128 in two rounds 36; 2176 x 7680 on 128 x 256 64,
 // 64 x 128 over 75; 2176 x 12288 on 256 x 256 104, 128 x 256 over 110.
 struct TileCost {
-    int bm, bn, per_cu;
+    int lm, ln, per_cu;   // log2 of the tile's rows and columns
     double t1, t2, fixed;
 };
 constexpr TileCost kTile[kTiles] = {
-    {32, 64, 2, 0.200, 0.280, 3.0},   {32, 128, 2, 0.226, 0.360, 3.0}, {64, 64, 2, 0.207, 0.300, 3.5},
-    {64, 128, 2, 0.280, 0.470, 3.0},  {64, 256, 1, 0.470, 0.470, 3.5}, {128, 128, 1, 0.470, 0.470, 4.0},
-    {128, 256, 1, 0.580, 0.580, 6.0}, {256, 256, 1, 1.020, 1.020, 10.0}};
+    {5, 6, 2, 0.200, 0.280, 3.0}, {5, 7, 2, 0.226, 0.360, 3.0}, {6, 6, 2, 0.207, 0.300, 3.5},
+    {6, 7, 2, 0.280, 0.470, 3.0}, {6, 8, 1, 0.470, 0.470, 3.5}, {7, 7, 1, 0.470, 0.470, 4.0},
+    {7, 8, 1, 0.580, 0.580, 6.0}, {8, 8, 1, 1.020, 1.020, 10.0}};
 constexpr double kOperandRate = 14.2e6, kStoreRate = 5e6;   // bytes per us
 // a separate kernel launch, and its rate over the bytes it moves
 constexpr double kLaunch = 3.5, kPassRate = 5e6;
 
+// (shifts and products by constants: a plan is worked out on the host for every launch)
 double tile_us(const TileCost& c, int64_t tiles, int KT, int splits) {
-    const int64_t n = tiles * splits, slots = (int64_t)256 * c.per_cu;
-    const int kt = (KT + splits - 1) / splits;
+    const int64_t n = tiles * splits;
+    const int ls = c.per_cu == 2 ? 9 : 8;   // log2 of the resident slots
+    const int kt = splits == 1 ? KT : (int)((unsigned)(KT + splits - 1) / (unsigned)splits);
+    const double bytes = (double)((1 << c.lm) + (1 << c.ln)) * (128 / kOperandRate);
+    const double out = c.per_cu == 1 ? (double)(1 << (c.lm + c.ln)) * (4 / kStoreRate) : 0.0;
     auto round = [&](int64_t w) {
-        const double t = std::max(w > 256 ? c.t2 : c.t1, (double)w * (c.bm + c.bn) * 128 / kOperandRate);
-        const double st = c.per_cu == 1 ? (double)w * c.bm * c.bn * 4 / kStoreRate : 0.0;
-        return kt * t + c.fixed + st;
+        return kt * std::max(w > 256 ? c.t2 : c.t1, (double)w * bytes) + c.fixed + (double)w * out;
     };
-    if (n <= slots) return round(n);
+    if (n <= (int64_t)1 << ls) return round(n);
     // two workgroups per CU drift apart, so a partly filled last round overlaps the one before it
-    if (c.per_cu > 1) return round(slots) * ((double)n / (double)slots + 0.3);
-    const int64_t full = n / slots, rest = n - full * slots;
-    return (double)full * round(slots) + (rest ? round(rest) : 0.0);
+    if (c.per_cu > 1) return round(512) * ((double)n * (1.0 / 512) + 0.3);
+    const int64_t full = n >> ls, rest = n & 255;
+    return (double)full * round(256) + (rest ? round(rest) : 0.0);
 }
 
 // The cheapest tile and split count of a bf16 Mt x Nt x K product under tile_us. A split pays for its
@@ -421,22 +423,21 @@ TilePlan pick_plan(const sa3k_ctx* ctx, int64_t Mt, int64_t Nt, int64_t K, bool 
     double best_us = 1e30;
     for (int i = 0; i < kTiles; ++i) {
         const TileCost& c = kTile[i];
-        if (Mt <= 32 ? c.bm != 32 : c.bm == 32) continue;   // 32-row tiles where one holds every row
+        if (Mt <= 32 ? c.lm != 5 : c.lm == 5) continue;   // 32-row tiles where one holds every row
         if (i == T256x256 && !big) continue;
-        const int64_t tiles = ceil_div(Mt, c.bm) * ceil_div(Nt, c.bn), slots = (int64_t)256 * c.per_cu;
+        const int64_t tiles = ((Mt + (1 << c.lm) - 1) >> c.lm) * ((Nt + (1 << c.ln) - 1) >> c.ln), slots = 256 * c.per_cu;
         const int most = ctx->gemm_split && KT >= 16 && tiles < slots
                              ? (int)std::min<int64_t>({(int64_t)16, KT / 4, slots / tiles}) : 1;
-        double us_one = -1;
-        // unsplit, split until the slots are full, and half of that (each call works this out anew: the
-        // estimate has to stay well below a launch's own host time)
-        for (const int s : {1, most / 2, most}) {
-            if (s < 1 || (s == 1 && us_one >= 0)) continue;
-            const bool fused = s == 1 && c.bn == 256;
+        // unsplit, split until the slots are full, and half of that
+        const int counts[3] = {1, most / 2, most};
+        for (int k = 0; k < (most > 1 ? 3 : 1); ++k) {
+            const int s = counts[k];
+            if (k && s < 2) continue;
+            const bool fused = s == 1 && c.ln == 8;
             double us = tile_us(c, tiles, KT, s);
-            if (s > 1) us += kLaunch + s * out * 8 / kPassRate;
-            if (swiglu && !fused) us += kLaunch + out * 8 / kPassRate;
-            if (heads && !(fused && c.bm != 256)) us += kLaunch + out * 10 / kPassRate;
-            if (s == 1) us_one = us;
+            if (s > 1) us += kLaunch + s * out * (8 / kPassRate);
+            if (swiglu && !fused) us += kLaunch + out * (8 / kPassRate);
+            if (heads && !(fused && c.lm != 8)) us += kLaunch + out * (10 / kPassRate);
             if (us < best_us) {
                 best_us = us;
                 best = TilePlan{(TileId)i, s};
