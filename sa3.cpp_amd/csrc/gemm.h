@@ -136,8 +136,8 @@ struct GemmDesc {
     bf16* sw_g = nullptr;
     int64_t sw_ldg = 0;
     int* sw_done = nullptr;
-    // Per-head q/k preparation (HeadPrep; parts 0: off) where the chosen tiles allow it (bf16
-    // 128 x 256 tiles, no split over K, the staged epilogue, dim a multiple of 256); *hp_done is
+    // Per-head q/k preparation (HeadPrep; parts 0: off) where the chosen tiles allow it (bf16 64 or
+    // 128 x 256 ones, no split over K, the staged epilogue, dim a multiple of 256); *hp_done is
     // set then (else the caller prepares the heads itself). C and every other output unchanged.
     HeadPrep hp;
     int* hp_done = nullptr;

@@ -586,8 +586,8 @@ __device__ inline void staged_store(const DmaParams& p, const float* st, int64_t
     }
 }
 
-// HP: the per-head q/k preparation instantiation (128 x 256 bf16 tiles): the staged epilogue takes
-// the tile in two passes of 64 rows and keeps the tile rows' RoPE table rows in LDS past them.
+// HP: the per-head q/k preparation instantiation (256-column bf16 tiles): the staged epilogue takes
+// the tile in passes of 64 rows and keeps the tile rows' RoPE table rows in LDS past them.
 // XE: the instantiation that also runs the backward epilogues (DmaParams::ad / sb); the others do
 // not carry their code, which costs registers.
 // PLAIN: the instantiations whose operands all load through buffer descriptors (plain_ok); 2: with
