@@ -14,6 +14,7 @@
 #pragma once
 
 #include "gemm.h"
+#include "gemm_plan.h"
 #include "headprep.h"
 
 #include <algorithm>
@@ -78,7 +79,7 @@ struct DmaParams {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kRow = 128;   // LDS bytes per tile row
+constexpr int kRow = kTileRowBytes;   // LDS bytes per tile row
 
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
@@ -1292,10 +1293,10 @@ void launch_dma(sa3k_ctx* ctx, DmaParams p, int chosen = 0) {
     const int64_t grid = ceil_div(tiles, 8) * 8;
     const int KT = (int)(p.K / (BF16 ? 64 : 32));
     // resident workgroups per CU: as many as the 160 KiB of LDS hold (or the context's override)
-    constexpr int kLdsBytes = STAGES * (BM + BN) * kRow + 64;
-    const int wg_per_cu = ctx->gemm_wg_per_cu > 0 ? ctx->gemm_wg_per_cu : std::max(1, (160 * 1024) / kLdsBytes);
+    constexpr int kFit = dma_wg_per_cu(BM, BN, STAGES);
+    const int wg_per_cu = ctx->gemm_wg_per_cu > 0 ? ctx->gemm_wg_per_cu : kFit;
     const int64_t slots = (int64_t)256 * wg_per_cu;
-    static_assert((int64_t)256 * std::max(1, (160 * 1024) / kLdsBytes) * BM * BN <= kMaxSplitFloats,
+    static_assert((int64_t)256 * kFit * BM * BN <= kMaxSplitFloats,
                   "split partials of this tile family exceed kMaxSplitFloats");
     const int splits = split_count(ctx, tiles, slots, KT, &p.kps, chosen);
     p.ws = nullptr;
@@ -1394,12 +1395,6 @@ void launch_dma(sa3k_ctx* ctx, DmaParams p, int chosen = 0) {
 void gemm_launch_big(sa3k_ctx* ctx, DmaParams p, int chosen);
 void gemm_launch_wide(sa3k_ctx* ctx, const DmaParams& p, int chosen);
 
-// The tiles a bf16 product is cut into (gemm_dma.hip chooses, gemm_plan.hip launches)
-enum TileId { T32x64, T32x128, T64x64, T64x128, T64x256, T128x128, T128x256, T256x256, kTiles };
-struct TilePlan {
-    TileId tile;
-    int splits;
-};
 void gemm_launch_plan(sa3k_ctx* ctx, const DmaParams& p, const TilePlan& t);
 
 }  // namespace sa3k

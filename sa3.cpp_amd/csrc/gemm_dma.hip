@@ -308,6 +308,7 @@ void gemm_launch_big(sa3k_ctx* ctx, DmaParams p, int chosen) {
     const int64_t grid = ceil_div(tiles, 8) * 8;
     const int KT = (int)(p.K / 64);
     const int64_t slots = 256;   // one workgroup per CU (128 KiB of LDS)
+    static_assert(kTile[T256x256].per_cu() == 1, "the plan's slots of the 256 x 256 tiles");
     static_assert((int64_t)256 * 256 * 256 <= kMaxSplitFloats, "256 x 256 split partials exceed kMaxSplitFloats");
     const int splits = split_count(ctx, tiles, slots, KT, &p.kps, chosen);
     p.ws = nullptr;
@@ -371,83 +372,6 @@ bool plain_ok(const DmaParams& p) {
     return p.K2 == 0 || (fits(p.M, p.lda2, p.K2) && fits(p.N, p.ldb2, p.K2));
 }
 
-// ---- the bf16 tile and split choice
-// What a bf16 launch is estimated to take, in us, from what its tiles measured on MI355X (f32
-// output, K 768 to 12288, 77 to 4096 rows): per K tile of 64 a resident workgroup takes t1 alone on
-// its CU and t2 beside a second one, and all of them together no less than their operand bytes at
-// kOperandRate, the rate at which the caches feed the CUs' DMA. A round adds `fixed` for the launch, the first tile's latency and a lone epilogue.
-// One workgroup per CU leaves the output stores of a round exposed (kStoreRate); two hide them behind
-// each other's products. What the choice is about, K 1536: 343 x 1536 on 64 x 64 tiles 9.4 us, split
-// in 6 on 128 x 128 with its reduction 16.9; 343 x 4608 on 64 x 128 12.2, 128 x 128 split in 2 21.7;
-// 279 x 12288 on 64 x 256 or 128 x 256 20, 128 x 128 in two rounds 36; 2176 x 7680 on 128 x 256 64,
-// 64 x 128 over 75; 2176 x 12288 on 256 x 256 104, 128 x 256 over 110.
-struct TileCost {
-    int lm, ln, per_cu;   // log2 of the tile's rows and columns
-    double t1, t2, fixed;
-};
-constexpr TileCost kTile[kTiles] = {
-    {5, 6, 2, 0.200, 0.280, 3.0}, {5, 7, 2, 0.226, 0.360, 3.0}, {6, 6, 2, 0.207, 0.300, 3.5},
-    {6, 7, 2, 0.280, 0.470, 3.0}, {6, 8, 1, 0.470, 0.470, 3.5}, {7, 7, 1, 0.470, 0.470, 4.0},
-    {7, 8, 1, 0.580, 0.580, 6.0}, {8, 8, 1, 1.020, 1.020, 10.0}};
-constexpr double kOperandRate = 14.2e6, kStoreRate = 5e6;   // bytes per us
-// a separate kernel launch, and its rate over the bytes it moves
-constexpr double kLaunch = 3.5, kPassRate = 5e6;
-
-// (shifts and products by constants: a plan is worked out on the host for every launch)
-double tile_us(const TileCost& c, int64_t tiles, int KT, int splits) {
-    const int64_t n = tiles * splits;
-    const int ls = c.per_cu == 2 ? 9 : 8;   // log2 of the resident slots
-    const int kt = splits == 1 ? KT : (int)((unsigned)(KT + splits - 1) / (unsigned)splits);
-    const double bytes = (double)((1 << c.lm) + (1 << c.ln)) * (128 / kOperandRate);
-    const double out = c.per_cu == 1 ? (double)(1 << (c.lm + c.ln)) * (4 / kStoreRate) : 0.0;
-    auto round = [&](int64_t w) {
-        return kt * std::max(w > 256 ? c.t2 : c.t1, (double)w * bytes) + c.fixed + (double)w * out;
-    };
-    if (n <= (int64_t)1 << ls) return round(n);
-    // two workgroups per CU drift apart, so a partly filled last round overlaps the one before it
-    if (c.per_cu > 1) return round(512) * ((double)n * (1.0 / 512) + 0.3);
-    const int64_t full = n >> ls, rest = n & 255;
-    return (double)full * round(256) + (rest ? round(rest) : 0.0);
-}
-
-// The cheapest tile and split count of a bf16 Mt x Nt x K product under tile_us. A split pays for its
-// partial sums and their reduction launch; tiles that cannot run an epilogue the caller asks for (the
-// paired SwiGLU and the head preparation need 256 columns, the latter not 256 rows, and neither a
-// split) pay for the separate kernel that replaces it. The layout of B has no say, so both layouts of
-// one product sum alike. big: whether 256 x 256 tiles may be used.
-TilePlan pick_plan(const sa3k_ctx* ctx, int64_t Mt, int64_t Nt, int64_t K, bool big, bool swiglu, bool heads,
-                   double* est = nullptr) {
-    const int KT = (int)(K / 64);
-    const double out = (double)Mt * (double)Nt;
-    TilePlan best{T128x256, 1};
-    double best_us = 1e30;
-    for (int i = 0; i < kTiles; ++i) {
-        const TileCost& c = kTile[i];
-        if (Mt <= 32 ? c.lm != 5 : c.lm == 5) continue;   // 32-row tiles where one holds every row
-        if (i == T256x256 && !big) continue;
-        const int64_t tiles = ((Mt + (1 << c.lm) - 1) >> c.lm) * ((Nt + (1 << c.ln) - 1) >> c.ln), slots = 256 * c.per_cu;
-        const int most = ctx->gemm_split && KT >= 16 && tiles < slots
-                             ? (int)std::min<int64_t>({(int64_t)16, KT / 4, slots / tiles}) : 1;
-        // unsplit, split until the slots are full, and half of that
-        const int counts[3] = {1, most / 2, most};
-        for (int k = 0; k < (most > 1 ? 3 : 1); ++k) {
-            const int s = counts[k];
-            if (k && s < 2) continue;
-            const bool fused = s == 1 && c.ln == 8;
-            double us = tile_us(c, tiles, KT, s);
-            if (s > 1) us += kLaunch + s * out * (8 / kPassRate);
-            if (swiglu && !fused) us += kLaunch + out * (8 / kPassRate);
-            if (heads && !(fused && c.lm != 8)) us += kLaunch + out * (10 / kPassRate);
-            if (us < best_us) {
-                best_us = us;
-                best = TilePlan{(TileId)i, s};
-            }
-        }
-    }
-    if (est) *est = best_us;
-    return best;
-}
-
 // the plan applies where no option asks for a particular tile family
 bool planned(const sa3k_ctx* ctx) {
     return ctx->gemm_small == 4 && (ctx->gemm_cfg == 0 || ctx->gemm_cfg == 4) && ctx->gemm_big == 3 && ctx->gemm_splits == 0 &&
@@ -476,7 +400,7 @@ namespace {
 void dispatch_dma_kn(sa3k_ctx* ctx, const DmaParams& p) {
     const int64_t Mt = p.Mp + p.Mx;
     if (planned(ctx) && p.N > 64 && plain_ok(p))
-        return gemm_launch_plan(ctx, p, pick_plan(ctx, Mt, p.Nt, p.K, big_ok(ctx, p) && vec_epi_ok(p), false, false));
+        return gemm_launch_plan(ctx, p, pick_plan(Mt, p.Nt, p.K, ctx->gemm_split, big_ok(ctx, p) && vec_epi_ok(p), false, false));
     if (use_big_tiles(ctx, Mt, p.N, p.K) && big_ok(ctx, p) && vec_epi_ok(p)) return gemm_launch_big(ctx, p, 0);
     if (Mt <= 32) return launch_dma<32, 128, 1, 4, true, 4, true>(ctx, p);
     if (p.N <= 64) return launch_dma<128, 64, 4, 4, true, 4, true>(ctx, p);
@@ -499,7 +423,7 @@ void dispatch_dma_dq(sa3k_ctx* ctx, const DmaParams& p) {
     // tile's resident workgroups go
     auto splits = [&](int bm, int bn, int64_t slots) {
         if (!planned(ctx) || p.N <= 64) return 0;
-        const int s = pick_plan(ctx, p.M, p.N, p.K, true, false, false).splits;
+        const int s = pick_plan(p.M, p.N, p.K, ctx->gemm_split, true, false, false).splits;
         return (int)std::max<int64_t>(1, std::min<int64_t>(s, slots / (ceil_div(p.M, bm) * ceil_div(p.N, bn))));
     };
     // (decoded B: the 64 x 128 tile, whose four waves side by side along N decode each fragment once)
@@ -513,8 +437,8 @@ template <bool BF16>
 void dispatch_dma(sa3k_ctx* ctx, const DmaParams& p) {
     if constexpr (BF16) {
         if (planned(ctx) && p.bq == 0 && !p.b_kn && p.Nt > 64 && plain_ok(p))
-            return gemm_launch_plan(ctx, p, pick_plan(ctx, p.Mp + p.Mx, p.Nt, p.K, big_ok(ctx, p) && vec_epi_ok(p),
-                                                        p.sw_half > 0, p.hp.parts > 0));
+            return gemm_launch_plan(ctx, p, pick_plan(p.Mp + p.Mx, p.Nt, p.K, ctx->gemm_split,
+                                                        big_ok(ctx, p) && vec_epi_ok(p), p.sw_half > 0, p.hp.parts > 0));
         // per-head q/k preparation: 128 x 256 tiles
         if (p.hp.parts > 0 && p.bq == 0 && !p.b_kn) return gemm_launch_wide(ctx, p, 0);
         if (p.bq == 1) return dispatch_dma_dq<1>(ctx, p);
@@ -595,8 +519,8 @@ bool gemm_extra_cols_free(const sa3k_ctx* ctx, int64_t Mt, int64_t N, int64_t K,
     // (a product of its own beside this one costs a launch and the streams' fork and join on the host)
     if (planned(ctx) && N > 64) {
         double without = 0, with = 0;
-        if (pick_plan(ctx, Mt, N, K, true, false, false, &without).tile < T128x256 &&
-            pick_plan(ctx, Mt, N + Nx, K, true, false, false, &with).tile < T128x256)
+        if (pick_plan(Mt, N, K, ctx->gemm_split, true, false, false, &without).tile < T128x256 &&
+            pick_plan(Mt, N + Nx, K, ctx->gemm_split, true, false, false, &with).tile < T128x256)
             return with <= without + 0.5;
     }
     return dma_rounds(ctx, Mt, N + Nx, K) <= dma_rounds(ctx, Mt, N, K);

@@ -319,6 +319,19 @@ def test_dora_odd_tokens(ctx, N):
             assert rel_err(got[k], ref[k]) < 2e-2 and cosine(got[k], ref[k]) >= 0.9999, (N, in_, out_, k)
 
 
+@pytest.mark.parametrize("N,in_,out_", [(1, 3072, 3072), (2, 4608, 2304), (3, 2304, 6144), (10, 2176, 9216)])
+def test_few_tokens_long_k(ctx, N, in_, out_):
+    """A few tokens through wide linears: the products split over K on 32-row tiles, forward and the
+    [K][N] dX, whose splits have to fit the workgroups that a CU's LDS holds. The bf16 bar against the
+    oracle."""
+    X, dY, W, A, B = make_inputs(47, N, in_, out_, 16)
+    Wh = W.astype(np.float16)
+    got = run_gpu(ctx, X, dY, Wh, sa3k.TYPE_F16, A, B, 1.25, False, None, sa3k.PREC_BF16)
+    ref = run_oracle(X, dY, Wh.astype(np.float32), A, B, 1.25, False, None)
+    for k in ("Y", "dX", "dA", "dB"):
+        assert rel_err(got[k], ref[k]) < 2e-2 and cosine(got[k], ref[k]) >= 0.9999, k
+
+
 @pytest.mark.parametrize("big", [0, 1, 2])
 def test_dx_k_major_operand(ctx, big):
     """Merged linears' dX product reads W + s B A in its stored [out][in] layout as a K-major B
