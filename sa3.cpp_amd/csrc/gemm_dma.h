@@ -73,7 +73,8 @@ struct DmaParams {
     AttnDot ad;           // the attention dO epilogue (GemmDesc::ad; doh null: off)
     SwiBwd sb;            // the SwiGLU backward epilogue (GemmDesc::sb; du null: off)
     int* bwd_done;        // host-side, like sw_done
-    int64_t Mp;           // tile-grid row where the extra rows start: M rounded up to 8 (without extra rows: M)
+    int64_t Mp;           // tile-grid row where the extra rows start: M rounded up to 8 where whole slots of 8 rows come
+                          // from one source (PLAIN, 256 x 256 tiles), else M; without extra rows: M
 };
 
 namespace {
@@ -253,6 +254,7 @@ __device__ __forceinline__ void dma16(const void* g, uint32_t lds_addr) {
     asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_addr), "v"(g) : "memory");
 }
 
+template <bool GAP = true>
 __device__ inline void epilogue_elem(const DmaParams& p, int64_t m, int64_t n, float acc) {
     if (n >= p.N) {   // extra column
         if (m < p.M) p.Cbn[m * p.ldcn + (n - p.N)] = (bf16)(p.alpha_x * acc);
@@ -260,12 +262,13 @@ __device__ inline void epilogue_elem(const DmaParams& p, int64_t m, int64_t n, f
     }
     float x = p.alpha * acc;
     if (m >= p.M) {
-        if (m < p.Mp) return;   // between the main and the extra rows
+        if (GAP && m < p.Mp) return;   // between the main and the extra rows
+        const int64_t xr = m - (GAP ? p.Mp : p.M);
         if (p.Cbx) {
-            p.Cbx[(m - p.Mp) * p.ldcx + n] = (bf16)x;
+            p.Cbx[xr * p.ldcx + n] = (bf16)x;
             return;
         }
-        float* cx = p.Cx + (m - p.Mp) * p.ldcx + n;
+        float* cx = p.Cx + xr * p.ldcx + n;
         *cx = p.accumulate_x ? *cx + x : x;
         return;
     }
@@ -325,6 +328,8 @@ __device__ inline float4 epi_scale(const DmaParams& p, float4 x, const EpiCols& 
 // Epilogue of four consecutive columns n..n+3 of row m (host-checked: 16-byte aligned rows, N a
 // multiple of 4), same operations and order as epilogue_elem; k = epi_cols(p, n). Returns the
 // main-row value before accumulation into C (unspecified for extra rows and columns).
+// GAP: the extra rows start at Mp, past a gap of rows that are not stored (else right at M).
+template <bool GAP = true>
 __device__ inline float4 epilogue_vec4(const DmaParams& p, int64_t m, int64_t n, float4 a, const EpiCols& k) {
     if (n >= p.N) {   // four extra columns (N % 4 == 0)
         if (m < p.M) {
@@ -336,13 +341,14 @@ __device__ inline float4 epilogue_vec4(const DmaParams& p, int64_t m, int64_t n,
     }
     float4 x = make_float4(p.alpha * a.x, p.alpha * a.y, p.alpha * a.z, p.alpha * a.w);
     if (m >= p.M) {
-        if (m < p.Mp) return x;
+        if (GAP && m < p.Mp) return x;
+        const int64_t xr = m - (GAP ? p.Mp : p.M);
         if (p.Cbx) {
             bf16 b[4] = {(bf16)x.x, (bf16)x.y, (bf16)x.z, (bf16)x.w};
-            *reinterpret_cast<uint2*>(p.Cbx + (m - p.Mp) * p.ldcx + n) = __builtin_bit_cast(uint2, b);
+            *reinterpret_cast<uint2*>(p.Cbx + xr * p.ldcx + n) = __builtin_bit_cast(uint2, b);
             return x;
         }
-        float4* cx = reinterpret_cast<float4*>(p.Cx + (m - p.Mp) * p.ldcx + n);
+        float4* cx = reinterpret_cast<float4*>(p.Cx + xr * p.ldcx + n);
         if (p.accumulate_x) {
             const float4 o = *cx;
             x = make_float4(o.x + x.x, o.y + x.y, o.z + x.z, o.w + x.w);
@@ -534,7 +540,7 @@ __device__ inline void swiglu_bwd_store(const DmaParams& p, int64_t m, int64_t n
 // floats per row): thread tid stores chunk column cq (output column nq, column factors kq) of tile
 // rows tid / CPR + i NT / CPR. With 256-column tiles a wave holds one row, which the paired SwiGLU
 // and the head preparation rely on.
-template <int BN, int NT, int ER, int EROW, bool HP, bool XE = false>
+template <int BN, int NT, int ER, int EROW, bool HP, bool XE = false, bool GAP = true>
 __device__ inline void staged_store(const DmaParams& p, const float* st, int64_t m0, int64_t n0, int rb, int64_t Mt,
                                     int z, int tid, int cq, int64_t nq, const EpiCols& kq, bool sw_tile, bool hp_tile,
                                     const HeadPrepLane& hl, const float* tabs) {
@@ -576,7 +582,7 @@ __device__ inline void staged_store(const DmaParams& p, const float* st, int64_t
             continue;
         }
         const bool main_row = m < p.M;
-        const float4 v = main_row && main_col ? epilogue_main4(p, er, dr, a, kq) : epilogue_vec4(p, m, nq, a, kq);
+        const float4 v = main_row && main_col ? epilogue_main4(p, er, dr, a, kq) : epilogue_vec4<GAP>(p, m, nq, a, kq);
         if (BN == 256 && sw_tile && main_row) swiglu_pair_store(p, gp + (int64_t)dr * p.sw_ldg, lo, v);
         if constexpr (HP)
             if (hp_tile && main_row) head_prep_store(p, hl, (int)m, hb, ht, nq, v, tabs + (rb + r) * p.hp.rope_dims, outp, rsp);
@@ -635,7 +641,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_dma_kernel(DmaParams p) {
     // inserts no waits of its own; the loop orders DMA and reads with vmcnt waits and barriers.
     __shared__ __attribute__((aligned(1024))) char lds[STAGES * STAGE_BYTES];
 
-    const int64_t Mt = p.Mp + p.Mx;
+    constexpr bool GAP = PLAIN != 0;
+    const int64_t Mp = GAP ? p.Mp : p.M;   // first extra row of the tile grid
+    const int64_t Mt = Mp + p.Mx;
     const int tiles_m = (int)((Mt + BM - 1) / BM), tiles_n = (int)((p.Nt + BN - 1) / BN);
     // This workgroup's item (split z, tile bid). Dispatch deals workgroups out to the 8 XCDs
     // round-robin in linear order (x fastest), so XCD c runs the linear ids L with L % 8 == c; it
@@ -675,10 +683,11 @@ __global__ __launch_bounds__(NW * 64) void gemm_dma_kernel(DmaParams p) {
     // kc = (s%8) ^ swz(row). Rows past the end re-read the last one (their results are never stored).
     //
     // Main-segment loads go through buffer descriptors when the operand extents allow it. a_src: 1
-    // every row of the tile from A, 2 every row from the extra rows Ax, 3 whole slots (8 rows per
-    // wave) from one or the other, 0 per-lane global addresses (as the second segment always uses).
+    // every row of the tile from A, 2 every row from the extra rows Ax, 0 per-lane global addresses
+    // (as the second segment always uses); 3, with PLAIN only: whole slots (8 rows per wave) from A
+    // or Ax.
     const bool use_buf = p.a_bytes != 0 && p.b_bytes != 0 && (p.Nx == 0 || p.bx_bytes != 0) && (p.Mx == 0 || p.ax_bytes != 0);
-    const int a_src = !use_buf ? 0 : (p.Mx == 0 || m0 + BM <= p.M) ? 1 : m0 >= p.Mp ? 2 : 3;
+    const int a_src = !use_buf ? 0 : (p.Mx == 0 || m0 + BM <= p.M) ? 1 : m0 >= Mp ? 2 : PLAIN != 0 ? 3 : 0;
     const u32x4 rs_a = buffer_rsrc(a_src == 2 ? p.Ax : p.A, a_src == 2 ? p.ax_bytes : p.a_bytes);
     const u32x4 rs_b = buffer_rsrc(p.B, p.b_bytes), rs_bx = buffer_rsrc(p.Bx, p.bx_bytes);
     uint32_t aoff[NA], boff[NB];
@@ -687,9 +696,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_dma_kernel(DmaParams p) {
     for (int q = 0; q < NA; ++q) {
         const int s = q * NT + tid, row = s >> 3, kc = (s & 7) ^ swz(row);
         const int64_t gm = min(m0 + row, Mt - 1);
-        aoff[q] = gm >= p.Mp ? (uint32_t)(((gm - p.Mp) * p.ldax + kc * CE) * EB)
+        aoff[q] = gm >= Mp ? (uint32_t)(((gm - Mp) * p.ldax + kc * CE) * EB)
                              : (uint32_t)((min(gm, p.M - 1) * p.lda + kc * CE) * EB);
-        if (a_src == 3 && min(m0 + (q * NT + wave * 64) / 8, Mt - 1) >= p.Mp) ax_mask |= 1u << q;
+        if (a_src == 3 && min(m0 + (q * NT + wave * 64) / 8, Mt - 1) >= Mp) ax_mask |= 1u << q;
     }
 #pragma unroll
     for (int q = 0; q < NB; ++q) {
@@ -698,36 +707,38 @@ __global__ __launch_bounds__(NW * 64) void gemm_dma_kernel(DmaParams p) {
         if (gn >= p.Nt) gn = 0;
         boff[q] = gn < p.N ? (uint32_t)((gn * p.ldb + kc * CE) * EB) : (uint32_t)(((gn - p.N) * p.ldbx + kc * CE) * EB);
     }
-    // The same chunks by global address, worked out where they are used: the paths that need them
-    // are rare, and 64-bit pointers kept over the K loop would cost the others registers. seg2: the
-    // second segment (a zero page past K2); t: K tile of the split.
-    auto a_ptr = [&](int q, bool seg2, int t) -> const char* {
-        int th = tid;
-        asm volatile("" : "+v"(th));   // not hoisted out of the K loop
-        const int s = q * NT + th, row = s >> 3, kc = (s & 7) ^ swz(row);
-        const int64_t g0 = min(m0 + row, Mt - 1), gm = min(g0, p.M - 1), xr = g0 - p.Mp;
-        if (seg2) {
-            if (kc * CE >= p.K2) return static_cast<const char*>(p.zero);
-            return xr < 0 ? static_cast<const char*>(p.A2) + (gm * p.lda2 + kc * CE) * EB
-                          : static_cast<const char*>(p.A2x) + (xr * p.lda2x + kc * CE) * EB;
+    // The same chunks by global address (second segment: a zero page past K2), worked out once: their
+    // 64-bit arithmetic at every use is 12-20 KB more code and spilled scalars in the K loop (f32: a
+    // 2048 x 9216 x 6144 product with a second segment 2281 us against 2094, a 46 x 32 x 960 one 11.0
+    // against 9.8)
+    constexpr int NPA = PLAIN == 0 ? NA : 0, NPB = PLAIN == 0 ? NB : 0;
+    const char *ag[NPA + 1], *a2g[NPA + 1], *bg[NPB + 1], *b2g[NPB + 1];
+#pragma unroll
+    for (int q = 0; q < NPA; ++q) {
+        const int s = q * NT + tid, row = s >> 3, kc = (s & 7) ^ swz(row);
+        const int64_t g0 = min(m0 + row, Mt - 1);
+        if (g0 < Mp) {
+            const int64_t gm = min(g0, p.M - 1);
+            ag[q] = static_cast<const char*>(p.A) + (gm * p.lda + k0 + kc * CE) * EB;
+            a2g[q] = kc * CE < p.K2 ? static_cast<const char*>(p.A2) + (gm * p.lda2 + kc * CE) * EB
+                                    : static_cast<const char*>(p.zero);
+        } else {
+            const int64_t xr = g0 - Mp;
+            ag[q] = static_cast<const char*>(p.Ax) + (xr * p.ldax + k0 + kc * CE) * EB;
+            a2g[q] = kc * CE < p.K2 ? static_cast<const char*>(p.A2x) + (xr * p.lda2x + kc * CE) * EB
+                                    : static_cast<const char*>(p.zero);
         }
-        const int64_t k = k0 + (int64_t)t * BKE + kc * CE;
-        return xr < 0 ? static_cast<const char*>(p.A) + (gm * p.lda + k) * EB
-                      : static_cast<const char*>(p.Ax) + (xr * p.ldax + k) * EB;
-    };
-    auto b_ptr = [&](int q, bool seg2, int t) -> const char* {
-        int th = tid;
-        asm volatile("" : "+v"(th));
-        const int s = q * NT + th, row = s >> 3, kc = (s & 7) ^ swz(row);
+    }
+#pragma unroll
+    for (int q = 0; q < NPB; ++q) {
+        const int s = q * NT + tid, row = s >> 3, kc = (s & 7) ^ swz(row);
         int64_t gn = tile_col_bn<BN>(p, n0, row);
         if (gn >= p.Nt) gn = 0;
-        if (seg2)
-            return kc * CE < p.K2 && gn < p.N ? static_cast<const char*>(p.B2) + (gn * p.ldb2 + kc * CE) * EB
-                                              : static_cast<const char*>(p.zero);
-        const int64_t k = k0 + (int64_t)t * BKE + kc * CE;
-        return gn < p.N ? static_cast<const char*>(p.B) + (gn * p.ldb + k) * EB
-                        : static_cast<const char*>(p.Bx) + ((gn - p.N) * p.ldbx + k) * EB;
-    };
+        bg[q] = gn < p.N ? static_cast<const char*>(p.B) + (gn * p.ldb + k0 + kc * CE) * EB
+                         : static_cast<const char*>(p.Bx) + ((gn - p.N) * p.ldbx + k0 + kc * CE) * EB;
+        b2g[q] = kc * CE < p.K2 && gn < p.N ? static_cast<const char*>(p.B2) + (gn * p.ldb2 + kc * CE) * EB
+                                            : static_cast<const char*>(p.zero);
+    }
     // the 8 rows of B slot (q, wave) start at n0 + (q * NT + 64 wave) / 8: one source per slot
     // (N % 8 == 0), chosen on the scalar unit
     unsigned bx_mask = 0;   // bit q: slot q's rows are extra columns (fixed over the K loop)
@@ -779,8 +790,6 @@ __global__ __launch_bounds__(NW * 64) void gemm_dma_kernel(DmaParams p) {
         rs_bs = buffer_rsrc(p.Bs, p.bs_bytes);
     }
 
-    // no slot of this wave reads extra rows or columns: every load's descriptor is fixed
-    const bool plain = (a_src == 1 || a_src == 2) && p.Nx == 0;
     // PLAIN: the second segment's loads, K2 valid columns of [rows][ld2] operands through their own
     // descriptors (chunks past K2 load zeros from beyond the extent); no extra rows beside it
     auto issue_seg2 = [&](uint32_t so_lds) {
@@ -828,23 +837,13 @@ __global__ __launch_bounds__(NW * 64) void gemm_dma_kernel(DmaParams p) {
             }
             return;
         }
-        if (BQ != 2 && plain && t < Tm) {
-#pragma unroll
-            for (int q = 0; q < NA; ++q) dma16b(rs_a, aoff[q], so, dst_a + q * NT * 16 + so_lds);
-#pragma unroll
-            for (int q = 0; q < NB; ++q) dma16b(rs_b, boff[q], sob, dst_b + q * NT * 16 + so_lds);
-        } else if (t < Tm) {
-            if (a_src == 3) {
-                const u32x4 rs_ax = buffer_rsrc(p.Ax, p.ax_bytes);
-#pragma unroll
-                for (int q = 0; q < NA; ++q)
-                    dma16b(pick_rsrc(((ax_mask >> q) & 1u) != 0, rs_ax, rs_a), aoff[q], so, dst_a + q * NT * 16 + so_lds);
-            } else if (a_src != 0) {
+        if (t < Tm) {
+            if (a_src != 0) {
 #pragma unroll
                 for (int q = 0; q < NA; ++q) dma16b(rs_a, aoff[q], so, dst_a + q * NT * 16 + so_lds);
             } else {
 #pragma unroll
-                for (int q = 0; q < NA; ++q) dma16(a_ptr(q, false, t), dst_a + q * NT * 16 + so_lds);
+                for (int q = 0; q < NA; ++q) dma16(ag[q] + (int64_t)t * (BKE * EB), dst_a + q * NT * 16 + so_lds);
             }
             if constexpr (BQ == 2) {   // quants, block scales, then the padding loads
                 const uint32_t kq = (uint32_t)(k0 + (int64_t)t * BKE);   // bytes into the quant rows
@@ -862,13 +861,13 @@ __global__ __launch_bounds__(NW * 64) void gemm_dma_kernel(DmaParams p) {
                     dma16b(pick_rsrc(slot_bx(q), rs_bx, rs_b), boff[q], slot_bx(q) ? sobx : sob, dst_b + q * NT * 16 + so_lds);
             } else {
 #pragma unroll
-                for (int q = 0; q < NB; ++q) dma16(b_ptr(q, false, t), dst_b + q * NT * 16 + so_lds);
+                for (int q = 0; q < NB; ++q) dma16(bg[q] + (int64_t)t * (BKE * EB), dst_b + q * NT * 16 + so_lds);
             }
         } else {
 #pragma unroll
-            for (int q = 0; q < NA; ++q) dma16(a_ptr(q, true, t), dst_a + q * NT * 16 + so_lds);
+            for (int q = 0; q < NA; ++q) dma16(a2g[q], dst_a + q * NT * 16 + so_lds);
 #pragma unroll
-            for (int q = 0; q < NB; ++q) dma16(b_ptr(q, true, t), dst_b + q * NT * 16 + so_lds);
+            for (int q = 0; q < NB; ++q) dma16(b2g[q], dst_b + q * NT * 16 + so_lds);
         }
     };
 
@@ -1081,7 +1080,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_dma_kernel(DmaParams p) {
             if (m >= Mt || n >= p.Nt) continue;
             float sum = 0.f;
             for (int zz = 0; zz < splits; ++zz) sum += ld_coherent(p.ws + (int64_t)zz * Mt * p.Nt + m * p.Nt + n);
-            epilogue_elem(p, m, n, sum);
+            epilogue_elem<GAP>(p, m, n, sum);
         }
         return;
     }
@@ -1098,7 +1097,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_dma_kernel(DmaParams p) {
                     const int64_t m = m0 + wm0 + MT * i + out_row(v);
                     if (m >= Mt) continue;
                     if (p.ws) p.ws[(int64_t)z * Mt * p.Nt + m * p.Nt + n] = acc[i][j][v];
-                    else epilogue_elem(p, m, n, acc[i][j][v]);
+                    else epilogue_elem<GAP>(p, m, n, acc[i][j][v]);
                 }
         }
         return;
@@ -1154,7 +1153,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_dma_kernel(DmaParams p) {
             }
         }
         __syncthreads();
-        staged_store<BN, NT, ER, EROW, HP, XE>(p, st, m0, n0, rb, Mt, z, tid, cq, nq, kq, sw_tile, hp_tile, hl, tabs);
+        staged_store<BN, NT, ER, EROW, HP, XE, GAP>(p, st, m0, n0, rb, Mt, z, tid, cq, nq, kq, sw_tile, hp_tile, hl, tabs);
         if (rb + ER < BM) __syncthreads();
     }
 }
@@ -1289,6 +1288,7 @@ void settle_bwd_epilogues(DmaParams& p, int splits, int bn) {
 template <int BM, int BN, int WMW, int STAGES, bool BF16, int NW = 4, bool KN = false, int BQ = 0, bool HP = false,
           int PLAIN = 0>
 void launch_dma(sa3k_ctx* ctx, DmaParams p, int chosen = 0) {
+    if (PLAIN == 0) p.Mp = p.M;   // extra rows right after the main ones
     const int64_t tiles = ceil_div(p.Mp + p.Mx, BM) * ceil_div(p.Nt, BN);
     const int64_t grid = ceil_div(tiles, 8) * 8;
     const int KT = (int)(p.K / (BF16 ? 64 : 32));
