@@ -415,22 +415,18 @@ void dispatch_dma_kn(sa3k_ctx* ctx, const DmaParams& p) {
 // bf16 dispatch, else 128 x 256 tiles with the 8 waves side by side along N (128 x 32 each), so
 // every B fragment is decoded by one wave only (measured on MI355X, 2176 x 6144 x 1536 over Q8_0:
 // 91.5 us against 107.5 us with 2 x 4 waves of 64 x 64, whose two wave rows decode each fragment);
-// option gemm_dq 2 keeps the 2 x 4 layout. Both sum every output in the same order.
+// option gemm_dq 2 keeps the 2 x 4 layout. Both sum every output in the same order. These tiles split
+// over K by their own rule (split_count): the planned count of the product over a bf16 copy belongs to
+// smaller tiles and leaves these on few CUs (512 x 1536 x 6144 over Q8_0: 24 of 256, 165 us against 50
+// split in 10; 2 x 7040 x 1728 37 against 20).
 template <int BQ>
 void dispatch_dma_dq(sa3k_ctx* ctx, const DmaParams& p) {
     const int64_t tiles128 = ceil_div(p.M, 128) * ceil_div(p.N, 128);
-    // the split the same product over the bf16 copy takes (so that both sum alike), as far as this
-    // tile's resident workgroups go
-    auto splits = [&](int bm, int bn, int64_t slots) {
-        if (!planned(ctx) || p.N <= 64) return 0;
-        const int s = pick_plan(p.M, p.N, p.K, ctx->gemm_split, true, false, false).splits;
-        return (int)std::max<int64_t>(1, std::min<int64_t>(s, slots / (ceil_div(p.M, bm) * ceil_div(p.N, bn))));
-    };
     // (decoded B: the 64 x 128 tile, whose four waves side by side along N decode each fragment once)
     if (tiles128 < 384 && p.K < 4096 && (ctx->gemm_small == 2 || ctx->gemm_small == 4))
-        return launch_dma<64, 128, 1, 3, true, 4, false, BQ>(ctx, p, splits(64, 128, 512));
-    if (ctx->gemm_dq == 2) return launch_dma<128, 256, 2, 3, true, 8, false, BQ>(ctx, p, splits(128, 256, 256));
-    return launch_dma<128, 256, 1, 3, true, 8, false, BQ>(ctx, p, splits(128, 256, 256));
+        return launch_dma<64, 128, 1, 3, true, 4, false, BQ>(ctx, p);
+    if (ctx->gemm_dq == 2) return launch_dma<128, 256, 2, 3, true, 8, false, BQ>(ctx, p);
+    return launch_dma<128, 256, 1, 3, true, 8, false, BQ>(ctx, p);
 }
 
 template <bool BF16>

@@ -108,6 +108,28 @@ def test_chain_matches_oracle(ctx, wname, chain):
     assert rel_err(Bp, rBp) < 1e-5 and Bp.shape == rBp.shape
 
 
+@pytest.mark.parametrize("N,in_,out_", [(512, 6144, 1536), (128, 6144, 6144), (343, 4096, 1536), (2, 1728, 7040)])
+def test_decoded_base_splits_its_own_tiles(ctx, N, in_, out_):
+    """A product over a base decoded in the loader runs on its own tiles, fewer than the chip has CUs
+    here: it splits over K until they are busy, whatever the same product over the working copy takes.
+    Both sum the same exact products in f32, in another order."""
+    g = rng(317)
+    w, _ = make_weight(ctx, g, out_, in_, sa3k.TYPE_Q8_0)
+    X = g.normal(0, 1, (N, in_)).astype(np.float32)
+    try:
+        y_copy, _ = run_chain(ctx, w, [], X)
+        w.drop_working_copy()
+        ctx.profile(True)
+        ctx.profile_reset()
+        y_dec, _ = run_chain(ctx, w, [], X)
+        rep = ctx.profile_report()
+    finally:
+        ctx.profile(False)
+        w.destroy()
+    assert rel_err(y_dec, y_copy) < 1e-5
+    assert rep.get("gemm_splitk_reduce", (0,))[0] == 1, sorted(rep)
+
+
 def test_chain_order_matters(ctx):
     g = rng(311)
     in_, out_, N = 512, 768, 128
