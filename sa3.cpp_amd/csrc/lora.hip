@@ -17,6 +17,7 @@
 //                       dA += 2s B^T diag(gn) W + 2s^2 (B^T diag(gn) B) A
 //                       dA += sdUB^T X                     (column reduction)
 #include "lora.h"
+#include "refresh_plan.h"
 
 #include <algorithm>
 #include <cmath>
@@ -1593,7 +1594,6 @@ __global__ __launch_bounds__(kThreads) void group_dora_terms_kernel(const PrepDe
 //     |W + s B A|^2 - |W|^2, so no cancellation against bnsq), and P = W_eff A^T on MFMA from the
 //     bf16 W_eff rows, which the backward's dB term 2 s gn P and the magnitude d = m / sqrt(nsq)
 //     need. The row sums are reduced in a fixed lane order: deterministic.
-constexpr int kMergeRows = 64;
 constexpr int kMergeEP = 72;   // bf16 row pitch of the staged W_eff chunks (144 bytes: 16-byte aligned rows)
 
 // stored element type of a merge launch: its raw bytes per element and its decode
@@ -1926,21 +1926,6 @@ PrepDesc prep_desc(sa3k_ctx* ctx, sa3k_lin* L, const float* A, const float* B, c
     return q;
 }
 
-// Column splits of a member's 64-row blocks, by the 64 x 64 chunks of the whole refresh: a workgroup
-// walks its chunks one after another, about 1.3 us each (a memory round trip and two barriers), so
-// below a chip full of workgroups (four per CU) the time is that walk's length. A group that fills
-// the chip by its rows alone is not split; at least kMergeMinChunks chunks stay with a workgroup.
-// Measured on MI355X, whole refresh unsplit -> split, us: a 1536-wide block's seven linears (one
-// launch) dora r32 117 -> 68, lora r16 111 -> 56; one linear, dora r32: 1536 x 6144 Q8_0 38 -> 21,
-// 1536 x 9216 f16 34 -> 23, 6144 x 1536 f16 107 -> 20. Slots 768 / 2048 and minima of 6 / 8 chunks
-// were within 5% or slower.
-constexpr int kMergeSlots = 1024, kMergeMinChunks = 4;
-int merge_splits(int64_t chunks, int64_t in) {
-    const int64_t nc = in / 64, per = std::max<int64_t>(kMergeMinChunks, ceil_div(chunks, kMergeSlots));
-    const int64_t s = ceil_div(nc, per);
-    return (int)ceil_div(nc, ceil_div(nc, s));   // no split without chunks
-}
-
 // one launch per stored element type present (blocks of other members exit at once)
 template <class SRC>
 void launch_merge(sa3k_ctx* ctx, const SRC& src, sa3k_lin* const* lins, int n, int blocks, int merge_blocks, int r,
@@ -1986,8 +1971,9 @@ bool lin_prepare_merged(sa3k_ctx* ctx, sa3k_lin* const* lins, int n, const float
     std::stable_sort(idx.begin(), idx.end(), [&](int a, int b) { return lins[a]->W->in > lins[b]->W->in; });
     PrepInline src{};
     src.n = n;
-    int64_t chunks = 0;
-    for (int i = 0; i < n; ++i) chunks += ceil_div(lins[i]->W->out, kMergeRows) * (lins[i]->W->in / 64);
+    std::vector<RefreshMember> shapes;
+    for (int i = 0; i < n; ++i) shapes.push_back({lins[i]->W->in, lins[i]->W->out});
+    const std::vector<int> splits = refresh_splits(shapes, dora != 0, stream_counters(ctx) ? kMaxFixupTiles : 0);
     int blocks = 0;
     bool split = false;
     for (int k = 0; k < n; ++k) {
@@ -1995,14 +1981,12 @@ bool lin_prepare_merged(sa3k_ctx* ctx, sa3k_lin* const* lins, int n, const float
         order[k] = lins[i];
         PrepDesc& q = src.ds[k];
         q = prep_desc(ctx, lins[i], A[i], B[i], dora ? mag[i] : nullptr, dora ? bnsq[i] : nullptr, true);
-        q.msplit = merge_splits(chunks, q.in);
-        if (dora && !stream_counters(ctx)) q.msplit = 1;
+        q.msplit = splits[i];
         split = split || q.msplit > 1;
         q.blk0[kStageMerge] = blocks;
         blocks += (int)ceil_div(q.out, kMergeRows) * q.msplit;
     }
     const int merge_blocks = blocks;
-    if (split && dora) SA3K_REQUIRE(merge_blocks <= kMaxFixupTiles, "column splits need an arrival counter per block");
     for (int k = 0; k < n; ++k) {
         src.ds[k].blk0[kStageConvert] = blocks;
         blocks += (int)(ceil_div(src.ds[k].in, 64) + ceil_div(src.ds[k].out, 64));
@@ -2089,17 +2073,17 @@ LinGroup* lin_group_create(sa3k_ctx* ctx, sa3k_lin* const* lins, int n, const fl
             std::vector<int> order(n);
             for (int i = 0; i < n; ++i) order[i] = i;
             std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return h[a].in > h[b].in; });
-            int64_t chunks = 0;
-            for (const PrepDesc& q : h) chunks += ceil_div(q.out, kMergeRows) * (q.in / 64);
+            std::vector<RefreshMember> shapes;
+            for (const PrepDesc& q : h) shapes.push_back({q.in, q.out});
+            const std::vector<int> splits = refresh_splits(shapes, dora != 0, kMaxFixupTiles);
             for (int i : order) {
-                h[i].msplit = merge_splits(chunks, h[i].in);
+                h[i].msplit = splits[i];
                 g->split |= h[i].msplit > 1;
                 h[i].blk0[kStageMerge] = (int)bm[kStageMerge].size();
                 bm[kStageMerge].insert(bm[kStageMerge].end(), (size_t)(ceil_div(h[i].out, kMergeRows) * h[i].msplit), i);
             }
             g->merge_blocks = (int)bm[kStageMerge].size();
             if (g->merged) {   // the conversion blocks ride behind the merge blocks of the same launch
-                SA3K_REQUIRE(!g->split || g->merge_blocks <= kMaxFixupTiles, "column splits need an arrival counter per block");
                 if (g->split && g->dora) g->part = dev_alloc<float>((int64_t)g->merge_blocks * kMergePart);
                 for (PrepDesc& q : h) q.blk0[kStageConvert] += g->merge_blocks;
                 bm[kStageMerge].insert(bm[kStageMerge].end(), bm[kStageConvert].begin(), bm[kStageConvert].end());

@@ -138,6 +138,39 @@ LOCAL_CASES = {"full_dora_local65_f16": ("full", True, 0, False, 65),
                "core_lora_local65_band_weighted_f16": ("core", False, 6, True, 65)}
 
 
+@pytest.mark.parametrize("dora", [True, False])
+def test_dit_refresh_of_many_wide_blocks(ctx, dora):
+    """120 blocks of width 64 with an FFN of 2048: split by columns, the merged refresh would take 9480
+    workgroups, more than dora has arrival counters, so it runs unsplit (lora needs none and is split).
+    Against the rank term as a second segment, which refreshes in launches of its own: loss and
+    gradients agree to the bf16 roundings of the operands (B starts at zero, so W + s B A = W)."""
+    cfg = dict(CFG, B=1, T=8, Ctx=4, dim=64, heads=1, inner=2048, depth=120, dora=dora)
+    g = np.random.Generator(np.random.Philox(77))
+    inputs = {"x_t": g.normal(0, 1, (1, 8, 64)), "target": g.normal(0, 1, (1, 8, 64)), "t": g.uniform(0, 1, 1),
+              "cross": g.normal(0, 1, (1, 4, 64)), "glob": g.normal(0, 1, (1, 64))}
+    got, tensors = [], {}
+    for merge in (1, 0):
+        ctx.set_option("lin_merge", merge)
+        d = sa3k.Dit(ctx, sa3k.dit_config(64, 64, 120, 1, 64, 4, 64, 2048), sa3k.TYPE_F16)
+        try:
+            for name, rows, cols, typ in d.tensors():
+                if name not in tensors:
+                    t = np.ones(rows * cols, np.float32) if name.endswith("gamma") else \
+                        g.normal(0, 0.02, rows * cols).astype(np.float32)
+                    tensors[name] = t.astype(np.float16) if typ == sa3k.TYPE_F16 else t
+                d.set_tensor(name, tensors[name])
+            d.setup(8, 16.0, dora, sa3k.SCOPE_CORE, 1, 8, 4)
+            d.adapters_init(3, 0.0)
+            up, _ = upload_inputs(ctx, inputs)
+            loss = d.accumulate(up["x_t"], up["target"], up["t"], up["cross"], up["glob"])
+            got.append((loss, d.arena(1).numpy()))
+        finally:
+            d.destroy()
+    (l1, g1), (l0, g0) = got
+    assert np.allclose(l1, l0, rtol=1e-3) and np.isfinite(g1).all() and np.abs(g1).max() > 0
+    assert rel_err(g1, g0) < 2e-2 and cosine(g1, g0) >= 0.9999
+
+
 @pytest.mark.parametrize("seed", SEEDS)
 @pytest.mark.parametrize("name", sorted(LOCAL_CASES))
 def test_dit_local_conditioning_vs_oracle(ctx, name, seed):
