@@ -21,7 +21,7 @@ void launch_plan(sa3k_ctx* ctx, const DmaParams& p, const TilePlan& t) {
         case T64x64: return launch_tile<T64x64, 2, 4, KN, PLAIN>(ctx, p, s);
         case T64x128: return launch_tile<T64x128, 2, 8, KN, PLAIN>(ctx, p, s);
         case T64x256:
-            if constexpr (!KN && PLAIN == 1)
+            if constexpr (!KN)   // with extra columns too: an adapted QKV or cross-query product carries them
                 if (p.hp.parts > 0) return launch_tile<T64x256, 1, 8, false, PLAIN, true>(ctx, p, s);
             return launch_tile<T64x256, 1, 8, KN, PLAIN>(ctx, p, s);
         case T128x128: return launch_tile<T128x128, 2, 8, KN, PLAIN>(ctx, p, s);

@@ -148,6 +148,43 @@ def test_block_epilogue_fusions_bitwise(ctx, S):
                 assert np.array_equal(res[15][k][t], res[fuse][k][t]), (fuse, f"{k}[{t}]")
 
 
+@pytest.mark.parametrize("dim,S,prep", [(1536, 279, 2), (1536, 343, 2), (768, 256, 1), (768, 700, 1)])
+def test_block_epilogue_fusions_few_rows_bitwise(ctx, dim, S, prep):
+    """The forward fusions at a few hundred rows, where the products take 64 x 256 (and 128 x 256) tiles
+    and carry the rank product as extra columns: bit for bit the separate kernels' results, and as few
+    launches of those as the tiles allow (prep: the head preparation of the context K/V and, at 1536,
+    of the cross queries, whose product takes 64 x 128 tiles)."""
+    assert_shipped_options(ctx)
+    heads, Ctx = dim // 64, 77
+    print(f"epilogue fusions: dim {dim}, S {S}", flush=True)
+    cfg, w, x, cx, gc = bb.random_block(67, B=1, S=S, Ctx=Ctx, dim=dim, heads=heads, inner=4 * dim, rank=16,
+                                        alpha=16.0, dora=True, window=0, w_sd=0.02, b_sd=0.01)
+    dout = rng(68).normal(0, 1e-2, x.shape).astype(np.float32)
+    gb = GpuBlock(ctx, cfg, w, sa3k.TYPE_F16, S, Ctx)
+    res, launches = {}, {}
+    try:
+        for fuse in (0, 1, 2, 3):
+            ctx.set_option("epi_fuse", fuse)
+            ctx.profile(True)
+            ctx.profile_reset()
+            res[fuse] = run_gpu(ctx, gb, x, cx, gc, dout)
+            rep = ctx.profile_report()
+            ctx.profile(False)
+            launches[fuse] = tuple(sum(v[0] for k, v in rep.items() if k.startswith(n))
+                                   for n in ("blk_swiglu", "blk_prep_fwd"))
+    finally:
+        ctx.profile(False)
+        ctx.set_options(ctx.defaults)
+        gb.destroy()
+    assert launches == {f: (1 if f & 1 else 2, prep if f & 2 else 3) for f in launches}, launches
+    for fuse in (0, 1, 2):
+        for k in ("out", "dx", "dctx", "dgcond"):
+            assert np.array_equal(res[3][k], res[fuse][k]), (fuse, k)
+        for k in ("dA", "dB", "dm"):
+            for t in range(7):
+                assert np.array_equal(res[3][k][t], res[fuse][k][t]), (fuse, f"{k}[{t}]")
+
+
 @pytest.mark.parametrize("act_bf16", [1, 3])
 def test_block_fused_epilogues_vs_oracle(ctx, act_bf16):
     """The fused epilogues against the oracle directly: the full-width block at 2 x 136 tokens with
