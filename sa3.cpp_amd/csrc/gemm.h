@@ -160,9 +160,10 @@ struct GemmDesc {
 // any other source type the kernel that decodes it on its way into LDS (gemm.hip).
 void gemm_run(sa3k_ctx* ctx, const GemmDesc& d, const char* prof_name);
 void gemm_run_dma(sa3k_ctx* ctx, const GemmDesc& d);
-// whether Nx extra output columns ride on a bf16 Mt x N x K product without another round of
-// workgroups
-bool gemm_extra_cols_free(const sa3k_ctx* ctx, int64_t Mt, int64_t N, int64_t K, int64_t Nx);
+// whether Nx extra output columns on a bf16 Mt x N x K product (kn: B stored [K][N]; swiglu, heads: the
+// epilogues it is asked for) cost less than a product of their own beside it
+bool gemm_extra_cols_free(const sa3k_ctx* ctx, int64_t Mt, int64_t N, int64_t K, int64_t Nx, bool kn, bool swiglu,
+                          bool heads);
 // bf16 products with at most 32 output columns and a plain epilogue (gemm_skinny.hip)
 bool gemm_skinny_ok(const sa3k_ctx* ctx, const GemmDesc& d);
 void gemm_run_skinny(sa3k_ctx* ctx, const GemmDesc& d);

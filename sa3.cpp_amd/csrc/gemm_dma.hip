@@ -491,8 +491,9 @@ void dispatch_dma(sa3k_ctx* ctx, const DmaParams& p) {
     }
 }
 
-// Rounds of resident workgroups a bf16 DMA GEMM of Mt x Nt x K takes under the dispatch above
-// (the tile and split choices, ignoring operand alignment): splits x tiles / slots, rounded up.
+// Rounds of resident workgroups a bf16 DMA GEMM of Mt x Nt x K takes on the tile families of the
+// dispatch above that do not go by estimated time (options that force one, a [K][N] B with extra
+// columns), ignoring operand alignment: splits x tiles / slots, rounded up.
 int64_t dma_rounds(const sa3k_ctx* ctx, int64_t Mt, int64_t Nt, int64_t K) {
     const int KT = (int)(K / 64);
     auto rounds = [&](int64_t tiles, int64_t slots) {
@@ -509,16 +510,9 @@ int64_t dma_rounds(const sa3k_ctx* ctx, int64_t Mt, int64_t Nt, int64_t K) {
 
 }  // namespace
 
-// Whether Nx extra output columns ride on a bf16 Mt x N x K product without costing it another
-// round of workgroups (their tiles fill slots the product leaves idle).
-bool gemm_extra_cols_free(const sa3k_ctx* ctx, int64_t Mt, int64_t N, int64_t K, int64_t Nx) {
-    // (a product of its own beside this one costs a launch and the streams' fork and join on the host)
-    if (planned(ctx) && N > 64) {
-        double without = 0, with = 0;
-        if (pick_plan(Mt, N, K, ctx->gemm_split, true, false, false, &without).tile < T128x256 &&
-            pick_plan(Mt, N + Nx, K, ctx->gemm_split, true, false, false, &with).tile < T128x256)
-            return with <= without + 0.5;
-    }
+bool gemm_extra_cols_free(const sa3k_ctx* ctx, int64_t Mt, int64_t N, int64_t K, int64_t Nx, bool kn, bool swiglu,
+                          bool heads) {
+    if (planned(ctx) && !kn && N > 64) return extra_cols_pay(Mt, N, K, Nx, ctx->gemm_split, swiglu, heads);
     return dma_rounds(ctx, Mt, N + Nx, K) <= dma_rounds(ctx, Mt, N, K);
 }
 

@@ -105,4 +105,24 @@ inline TilePlan pick_plan(int64_t Mt, int64_t Nt, int64_t K, bool split, bool bi
     return best;
 }
 
+// What a bf16 product of M rows with at most 32 columns takes in launches of its own, in us: it streams
+// its M x K operand at about 1 TB/s (measured on MI355X: 2176 x 32 x 1536 11.6, 2176 x 32 x 6144 42.7 with
+// the reduction of its splits, which it needs past K 3072)
+constexpr double kRankRate = 1e6;
+inline double rank_product_us(int64_t M, int64_t K) {
+    return kLaunch * (K > 3072 ? 2 : 1) + (double)M * (double)K * (2 / kRankRate);
+}
+
+// Whether Nx columns cost a bf16 M x N x K product less as extra output columns than as a product of
+// their own, which runs beside it on the second stream at best, on the same CUs. Measured on MI355X
+// against columns only where they cost at most 0.5 us: the DiT update (24 blocks of 1536, 2176 rows) 32.07
+// -> 31.90 ms, 8 rank products a block instead of 11; the velocity of four such blocks, 1024 frames 1753
+// -> 1679 us, 512 frames 1338 -> 1290. Charging a half or a fifth of the product measured the same.
+inline bool extra_cols_pay(int64_t M, int64_t N, int64_t K, int64_t Nx, bool split, bool swiglu, bool heads) {
+    double without = 0.0, with = 0.0;
+    pick_plan(M, N, K, split, true, swiglu, heads, &without);
+    pick_plan(M, N + Nx, K, split, true, swiglu, heads, &with);
+    return with <= without + rank_product_us(M, K);
+}
+
 }  // namespace sa3k

@@ -921,9 +921,10 @@ void lin_forward_t(sa3k_ctx* ctx, sa3k_lin* L, int x_src, const void* X, int64_t
         X = L->Xb;
         x_src = SRC_BF16;
     }
-    // merged: Hc = s X A^T as r extra output columns of the main product (B rows from A) when they
-    // cost it no extra round of workgroups, else as its own product beside it
-    const bool h_cols = merged && bf && (ctx->rank_cols & 1) && gemm_extra_cols_free(ctx, N, W->out, W->in, L->rank);
+    // merged: Hc = s X A^T as r extra output columns of the main product (B rows from A) when that
+    // costs less than its own product beside it
+    const bool h_cols = merged && bf && (ctx->rank_cols & 1) &&
+                        gemm_extra_cols_free(ctx, N, W->out, W->in, L->rank, false, epi && epi->sw_g, epi && epi->hp);
     // Hc = s X A^T
     if (L->rank > 0 && !h_cols) {
         GemmDesc h;
@@ -1117,7 +1118,7 @@ void lin_backward_t(sa3k_ctx* ctx, sa3k_lin* L, int x_src, const void* X, int64_
     // (with W_eff read as a [K][N] operand the extra columns read B itself, [out][r], as a [K][Nx]
     // operand: whole 64-column sub-tiles of dX's columns, in % 64 == 0)
     const bool sdub_cols = merged && dX && (L->Wmt || (in % 64 == 0 && r % 8 == 0)) && (ctx->rank_cols & 2) &&
-                           gemm_extra_cols_free(ctx, N + (L->dora ? r : 0), in, out, r);
+                           gemm_extra_cols_free(ctx, N + (L->dora ? r : 0), in, out, r, !L->Wmt, false, false);
     // 4a. dA += sdUB^T X: the column-reduction partials only need sdUB and X, so they run before
     //     (on the second stream: beside) the dX GEMM; their sum is added to dA after the GEMM's
     //     extra dA rows (step 3), keeping the accumulation order of dA fixed. When the partials

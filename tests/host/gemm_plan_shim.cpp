@@ -14,4 +14,10 @@ double plan(int64_t M, int64_t N, int64_t K, int split, int big, int swiglu, int
     out[3] = p.splits;
     return est;
 }
+
+// whether cols extra columns ride on the product; *own: what they take in launches of their own, us
+int cols_pay(int64_t M, int64_t N, int64_t K, int64_t cols, int swiglu, int heads, double* own) {
+    *own = sa3k::rank_product_us(M, K);
+    return sa3k::extra_cols_pay(M, N, K, cols, true, swiglu != 0, heads != 0);
+}
 }

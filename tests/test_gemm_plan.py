@@ -22,6 +22,7 @@ def host(tmp_path_factory):
     L = C.CDLL(out)
     i64, i = C.c_int64, C.c_int
     L.plan.restype, L.plan.argtypes = C.c_double, [i64, i64, i64, i, i, i, i, C.POINTER(i)]
+    L.cols_pay.restype, L.cols_pay.argtypes = i, [i64, i64, i64, i64, i, i, C.POINTER(C.c_double)]
     return L
 
 
@@ -55,3 +56,22 @@ def test_splits_fit_the_resident_workgroups(host):
         assert s == 1 or s * tiles <= slots, (M, N, K, rows, cols, s)
         assert 1 <= s <= max(1, K // 64 // 4)
         assert plan(host, M, N, K, split=0)[3] == 1
+
+
+# the forward products of a block of width d: (outputs, inputs, paired SwiGLU, heads prepared)
+def block_products(d):
+    return {"qkv": (5 * d, d, 0, 1), "out": (d, d, 0, 0), "cross.q": (2 * d, d, 0, 1), "cross.out": (d, d, 0, 0),
+            "ff.proj": (8 * d, d, 1, 0), "ff.out": (d, 4 * d, 0, 0)}
+
+
+def test_rank_columns_ride_where_they_cost_less_than_a_product(host):
+    """the benchmark's 2176 rows of width 1536: only the QKV product, which the columns would cost a round
+    of 128 x 256 tiles, leaves its rank product to launches of its own"""
+    own = C.c_double()
+    ride = {n: host.cols_pay(2176, N, K, 32, sw, h, C.byref(own)) for n, (N, K, sw, h) in block_products(1536).items()}
+    assert ride == {"qkv": 0, "out": 1, "cross.q": 1, "cross.out": 1, "ff.proj": 1, "ff.out": 1}
+    for M, N, K in sizes():
+        if N <= 64:
+            continue
+        ride = host.cols_pay(M, N, K, 16, 0, 0, C.byref(own))
+        assert ride == (plan(host, M, N + 16, K)[4] <= plan(host, M, N, K)[4] + own.value)
