@@ -31,7 +31,10 @@ struct TilePlan {
 // each other's products. What the choice is about, K 1536: 343 x 1536 on 64 x 64 tiles 9.4 us, split
 // in 6 on 128 x 128 with its reduction 16.9; 343 x 4608 on 64 x 128 12.2, 128 x 128 split in 2 21.7;
 // 279 x 12288 on 64 x 256 or 128 x 256 20, 128 x 128 in two rounds 36; 2176 x 7680 on 128 x 256 64,
-// 64 x 128 over 75; 2176 x 12288 on 256 x 256 104, 128 x 256 over 110.
+// 64 x 128 over 75; 2176 x 12288 on 256 x 256 104, 128 x 256 over 110. 64 x 128's t1 is what 132 to 144 of
+// them took at K 6144 (31 to 32.5 us); at 0.28 they were preferred there to 128 x 128 split in 3 (2176 x
+// 512, 700 x 1536, 343 x 3072: 26.7), and to 64 x 64 at 858 x 1024 x 1024 (9.9 against 8.0) or 128 x 7680 x
+// 1536 (11.6 against 9.3).
 struct TileCost {
     int lm, ln, stages;   // log2 of the tile's rows and columns, LDS stages
     double t1, t2, fixed;
@@ -43,7 +46,7 @@ struct TileCost {
 };
 constexpr TileCost kTile[kTiles] = {
     {5, 6, 4, 0.200, 0.280, 3.0}, {5, 7, 4, 0.226, 0.226, 3.0}, {6, 6, 4, 0.207, 0.300, 3.5},
-    {6, 7, 3, 0.280, 0.470, 3.0}, {6, 8, 3, 0.470, 0.470, 3.5}, {7, 7, 3, 0.470, 0.470, 4.0},
+    {6, 7, 3, 0.300, 0.470, 3.0}, {6, 8, 3, 0.470, 0.470, 3.5}, {7, 7, 3, 0.470, 0.470, 4.0},
     {7, 8, 3, 0.580, 0.580, 6.0}, {8, 8, 2, 1.020, 1.020, 10.0}};
 constexpr double kOperandRate = 14.2e6, kStoreRate = 5e6;   // bytes per us
 // a separate kernel launch, and its rate over the bytes it moves

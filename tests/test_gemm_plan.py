@@ -58,6 +58,13 @@ def test_splits_fit_the_resident_workgroups(host):
         assert plan(host, M, N, K, split=0)[3] == 1
 
 
+@pytest.mark.parametrize("M,N,K,tile", [(2176, 512, 6144, (128, 128)), (343, 3072, 6144, (128, 128)),
+                                        (700, 1536, 6144, (128, 128)), (867, 1152, 4544, (64, 64))])
+def test_long_products_on_few_tiles(host, M, N, K, tile):
+    """half a chip of 64 x 128 tiles walking a long K takes longer than split 128 x 128 or 64 x 64 ones"""
+    assert plan(host, M, N, K)[:2] == tile
+
+
 # the forward products of a block of width d: (outputs, inputs, paired SwiGLU, heads prepared)
 def block_products(d):
     return {"qkv": (5 * d, d, 0, 1), "out": (d, d, 0, 0), "cross.q": (2 * d, d, 0, 1), "cross.out": (d, d, 0, 0),
