@@ -455,12 +455,20 @@ void dispatch_dma(sa3k_ctx* ctx, const DmaParams& p) {
     const int64_t tiles128 = ceil_div(Mt, 128) * ceil_div(p.Nt, 128);
     if constexpr (BF16)
         if (tiles128 < 384 && ctx->gemm_small == 4) return launch_dma<128, 128, 2, 3, true, 8>(ctx, p);
-    // f32: bound by the f32 MFMA, so what counts is the busiest CU's share of the output. Where
-    // 64 x 128 tiles fill the CUs unevenly, 64 x 64 ones do better (measured on MI355X, 2048 x 1536 x
-    // 1536: 768 tiles of 64 x 64, three on each CU, 80 us; 384 of 64 x 128, two on half of them, 109 us).
+    // f32: bound by the f32 MFMA, so what counts is the busiest CU's share of the output. 64 x 64 tiles
+    // where 64 x 128 ones fill the CUs unevenly (measured on MI355X, 2048 x 1536 x 1536: 768 tiles of 64 x
+    // 64, three on each CU, 80 us; 384 of 64 x 128, two on half of them, 109 us; 1000 x 9216 x 6144 895
+    // against 1214 on split 128 x 128 tiles; none of 120 shapes of 77 to 4096 rows, 512 to 9216 columns
+    // and K 512 to 6144 slower by over 2%), and where the 128 x 128 ones, two to a CU, leave a last round
+    // part empty: a CU that gets two of its tiles makes it a full round, so their share is 8 64 x 64 tiles
+    // a round. An eighth less is asked for, and K 1024: 2048 x 9216 x 6144 (18 against 24) 1989 -> 1829
+    // us, an f32 lora linear of 2048 tokens, 6144 to 9216, forward and backward 4497 -> 3819; 4096 x 9216 x
+    // 1536 (36 against 40) would go 924 -> 949.
     if constexpr (!BF16) {
         const int64_t n128 = ceil_div(Mt, 64) * ceil_div(p.Nt, 128), n64 = ceil_div(Mt, 64) * ceil_div(p.Nt, 64);
-        if (ctx->gemm_small == 4 && ctx->gemm_cfg == 0 && n128 >= 256 && ceil_div(n64, 256) < 2 * ceil_div(n128, 256))
+        const int64_t share = ceil_div(n64, 256);
+        const bool part_round = tiles128 >= 512 && p.K >= 1024 && 8 * share <= 7 * 8 * ceil_div(tiles128, 512);
+        if (ctx->gemm_small == 4 && ctx->gemm_cfg == 0 && n128 >= 256 && (share < 2 * ceil_div(n128, 256) || part_round))
             return launch_dma<64, 64, 2, 3, false>(ctx, p);
     }
     if (tiles128 < 384 && p.K < (BF16 ? 4096 : 2048)) {

@@ -185,6 +185,26 @@ def test_f32_tiles(ctx, M, N, K):
     assert rel_err(got, A.astype(np.float64) @ W.astype(np.float64).T) < 1e-6 * max(1.0, (K / 64) ** 0.5)
 
 
+@pytest.mark.parametrize("M,N,K,tile", [(2048, 6144, 1024, "64,64,2,3"), (2040, 9200, 1024, "64,64,2,3"),
+                                        (4096, 9216, 1024, "128,128,2,2"), (2048, 6144, 512, "128,128,2,2")])
+def test_f32_part_rounds(ctx, M, N, K, tile):
+    # f32 products whose 128 x 128 tiles leave the last round part empty take 64 x 64 ones, unless many
+    # rounds or a short K make it not worth it; f32 accumulation error only
+    r = rng(M + N + K)
+    A = r.normal(0, 1, (M, K)).astype(np.float32)
+    W = r.normal(0, 0.02, (N, K)).astype(np.float32)
+    ctx.profile(True)
+    ctx.profile_reset()
+    try:
+        got = run(ctx, A, W, M, N, K, sa3k.PREC_F32, sa3k.TYPE_F32, sa3k.TYPE_F32)
+        rep = ctx.profile_report()
+    finally:
+        ctx.profile(False)
+    assert f"gemm_dma<{tile},f32>" in rep, sorted(rep)
+    rows = slice(0, M, 97)
+    assert rel_err(got[rows], A[rows].astype(np.float64) @ W.astype(np.float64).T) < 1e-6 * (K / 64) ** 0.5
+
+
 @pytest.mark.parametrize("M,N,K", [(2176, 12288, 1536), (2176, 6144, 1536), (300, 640, 256), (520, 1000, 192),
                                    (2176, 1536, 6144)])
 def test_big_tile_gemm(ctx, M, N, K):
