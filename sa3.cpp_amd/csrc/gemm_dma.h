@@ -598,9 +598,11 @@ __device__ inline void staged_store(const DmaParams& p, const float* st, int64_t
 // XE: the instantiation that also runs the backward epilogues (DmaParams::ad / sb); the others do
 // not carry their code, which costs registers.
 // PLAIN: the instantiations whose operands all load through buffer descriptors (plain_ok); 2: with
-// extra columns beside a [N][K] B, whose descriptor picks cost the others 10% at 64 x 64 tiles. Without the other load paths the K loop is a few hundred bytes of code: a
-// launch of few K tiles spends its time on instruction fetch as well, and the general instantiation's
-// loop alone is larger than what the instruction cache holds of it.
+// extra columns beside a [N][K] B. Only its tiles that hold extra columns pick a descriptor per load
+// (picked on every load it cost 64 x 64 tiles 10%), so the plan does not charge for it. Without the
+// other load paths the K loop is a few hundred bytes of code: a launch of few K tiles spends its time
+// on instruction fetch as well, and with them the loop alone is larger than what the instruction cache
+// holds of it.
 template <int BM, int BN, int WMW, int STAGES, bool BF16, int NW = 4, bool KN = false, int BQ = 0, bool HP = false,
           bool XE = false, int PLAIN = 0>
 __global__ __launch_bounds__(NW * 64) void gemm_dma_kernel(DmaParams p) {

@@ -446,9 +446,10 @@ void dispatch_dma(sa3k_ctx* ctx, const DmaParams& p) {
     if (Mt <= 32) return launch_dma<32, 128, 1, 4, BF16>(ctx, p);
     if (p.Nt <= 32) return launch_dma<128, 32, 4, 4, BF16>(ctx, p);
     if (p.Nt <= 64) return launch_dma<128, 64, 4, 4, BF16>(ctx, p);
-    // Grids of 128x128 tiles that leave a quarter of the two-per-CU slots idle. bf16: no split, on
-    // 128 x 128 tiles with eight waves in one workgroup per CU (three stages, 96 KiB), at any K
-    // (measured on MI355X: 2176 x 1536 x 1536 21.4 us against 23.6 us on 64 x 128 tiles and 31.1 us
+    // bf16 from here on: what the plan does not take (an option that forces a tile family, a second
+    // segment beside extra rows, operands past 4 GiB). Grids of 128x128 tiles that leave a quarter of
+    // the two-per-CU slots idle: no split, on 128 x 128 tiles with eight waves in one workgroup per CU
+    // (three stages, 96 KiB), at any K (measured on MI355X: 2176 x 1536 x 1536 21.4 us against 23.6 us on 64 x 128 tiles and 31.1 us
     // on the default tile split over K; 2176 x 1536 x 6144 67.7 against 71.1 us split over K; the
     // DiT update 34.56 against 35.16 ms with the short-K products alone, then 33.66 against 33.97 ms
     // with the long-K ones too). f32 with a short K: 64 x 128 tiles, no split.
@@ -479,7 +480,7 @@ void dispatch_dma(sa3k_ctx* ctx, const DmaParams& p) {
             default: break;
         }
     }
-    // bf16: 128 x 256 tiles, three stages in 144 KiB of LDS (one workgroup per CU), 16 waves of
+    // bf16: 128 x 256 tiles (the plan's too), three stages in 144 KiB of LDS (one workgroup per CU), 16 waves of
     // 64 x 32 (four per SIMD, to hide the DMA and LDS latency behind each other's MFMAs). Against
     // two 128 x 128 workgroups per CU the tile moves a quarter fewer operand bytes per flop through
     // the CU's vector-memory path, which the MFMA rate otherwise saturates (measured on MI355X at

@@ -110,7 +110,7 @@ def test_block_epilogue_fusions_bitwise(ctx, S):
     epilogues (bit 2) and the SwiGLU backward (the up-projection's dU) from the down-projection's dX
     epilogue (bit 3). 2 x 1024 tokens take the 128 x 256 DMA tiles without a split over K for the
     forward products, 2 x 1088 (the benchmark's 2176 tokens) the 256 x 256 tiles for the
-    up-projection; the out-projections' dX products take the small-grid 128 x 128 tiles, the
+    up-projection; the out-projections' dX products take 128 x 128 tiles, the
     down-projection's the 256 x 256 ones. Each fused path evaluates the same expressions per
     element, so every output and gradient agrees bit for bit; the profile shows which separate
     kernels ran (SwiGLU: one forward and one backward launch, each unless fused; head prep: self +
@@ -188,10 +188,10 @@ def test_block_epilogue_fusions_few_rows_bitwise(ctx, dim, S, prep):
 @pytest.mark.parametrize("act_bf16", [1, 3])
 def test_block_fused_epilogues_vs_oracle(ctx, act_bf16):
     """The fused epilogues against the oracle directly: the full-width block at 2 x 136 tokens with
-    every epilogue fusion on (epi_fuse 15) and the split over K and the small-grid tile switched
-    off, so that the up-projection, QKV and cross-query products and the out- and down-projections'
-    dX products take unsplit 128 x 256 tiles and the fusions apply (shipped, these small grids take
-    split or 64 x 128 tiles and the separate kernels, which the other full-width tests cover); the
+    every epilogue fusion on (epi_fuse 15) and the split over K and the tile plan (gemm_small 0)
+    switched off, so that the up-projection, QKV and cross-query products and the out- and
+    down-projections' dX products take unsplit 128 x 256 tiles and the fusions apply (shipped, some of
+    these take 64 x 64 or 64 x 128 tiles and the separate kernels, which the other full-width tests cover); the
     backward reading the bf16 copy of the FFN up-projection's output (act_bf16 1, the default) and
     also those of the QKV and cross-query outputs (3)."""
     B, S, Ctx = 2, 64 + 72, 128

@@ -319,6 +319,22 @@ def test_dora_odd_tokens(ctx, N):
             assert rel_err(got[k], ref[k]) < 2e-2 and cosine(got[k], ref[k]) >= 0.9999, (N, in_, out_, k)
 
 
+@pytest.mark.parametrize("merge", [True, False])
+@pytest.mark.parametrize("N,in_,out_", [(33, 1536, 1536), (343, 1536, 1536), (343, 768, 3072), (700, 512, 2048)])
+def test_planned_tiles_of_a_linear(ctx, N, in_, out_, merge):
+    """An adapted linear at the rows whose products take 64-row tiles: merged (rank columns beside the
+    forward, a [K][N] B and extra DoRA rows in dX) and with the rank term as a second segment of both.
+    The bf16 bar against the oracle."""
+    X, dY, W, A, B = make_inputs(53, N, in_, out_, 24)
+    Wh = W.astype(np.float16)
+    Wdec = Wh.astype(np.float32)
+    mag = (oracle.row_norms(Wdec) * 0.97).astype(np.float32)
+    got = run_gpu(ctx, X, dY, Wh, sa3k.TYPE_F16, A, B, 1.25, True, mag, sa3k.PREC_BF16, merge=merge)
+    ref = run_oracle(X, dY, Wdec, A, B, 1.25, True, mag)
+    for k in ("Y", "dX", "dA", "dB", "dm"):
+        assert rel_err(got[k], ref[k]) < 2e-2 and cosine(got[k], ref[k]) >= 0.9999, k
+
+
 @pytest.mark.parametrize("N,in_,out_", [(1, 3072, 3072), (2, 4608, 2304), (3, 2304, 6144), (10, 2176, 9216)])
 def test_few_tokens_long_k(ctx, N, in_, out_):
     """A few tokens through wide linears: the products split over K on 32-row tiles, forward and the
