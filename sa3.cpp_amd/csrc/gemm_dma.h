@@ -710,9 +710,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_dma_kernel(DmaParams p) {
         boff[q] = gn < p.N ? (uint32_t)((gn * p.ldb + kc * CE) * EB) : (uint32_t)(((gn - p.N) * p.ldbx + kc * CE) * EB);
     }
     // The same chunks by global address (second segment: a zero page past K2), worked out once: their
-    // 64-bit arithmetic at every use is 12-20 KB more code and spilled scalars in the K loop (f32: a
-    // 2048 x 9216 x 6144 product with a second segment 2281 us against 2094, a 46 x 32 x 960 one 11.0
-    // against 9.8)
+    // 64-bit arithmetic at every use is 12-24 KB more code and spilled scalars in the K loop (an f32 46 x
+    // 960 x 192 product with a second segment 15.9 us against 14.4, its rank product 11.0 against 9.5; the
+    // head preparation of 576 rows on 128 x 256 tiles 43.6 against 40.5)
     constexpr int NPA = PLAIN == 0 ? NA : 0, NPB = PLAIN == 0 ? NB : 0;
     const char *ag[NPA + 1], *a2g[NPA + 1], *bg[NPB + 1], *b2g[NPB + 1];
 #pragma unroll
